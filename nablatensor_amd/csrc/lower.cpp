@@ -1296,9 +1296,37 @@ class Emitter {
     int p = -1, r = -1;  // invariant nodes (p = -1: no offset)
     int s_kind = ARG_NONE, s_ref = -1;
     bool neg_p = false, neg_r = false;
+    bool linear = false;  // S comes from the sums of the draws, below
   };
   std::vector<GeoAffine> gaff_;  // per loop position (the carry)
   void plan_geo_affine();
+  // Such an s that is a linear form of the step's draws with literal
+  // coefficients (a correlated normal: a row of a Cholesky factor times the
+  // step's normals): the form of the draws' sums is the sum of the forms, so
+  // the loop adds up the draws alone and the step's nodes that only feed such
+  // exponents (hoist_) are evaluated once, after the loop, on those sums
+  // (hoisted_step). For a worst-of basket of 16 assets that takes the 136 fma
+  // of the step's 16 x 16 triangular map out of the loop: 2.55 -> 1.89 ms
+  // (fp32) and 6.63 -> 5.02 ms (fp64) per 10^6 paths of 252 steps. Taken when
+  // it saves at least kSumSaves instructions per step (the carries' sums and
+  // the map's sums against the draws to add); below that, a basket of two, the
+  // draws themselves are nearly all of the step. fp32 sums run over kSumSteps
+  // steps at a time and go to fp64 sums between (a conversion and an add per
+  // draw every kSumSteps steps, under 1 % of them): two assets' paths that end
+  // close to each other keep their order, which decides the asset a worst-of
+  // credits its derivatives to.
+  static constexpr int kSumSaves = 4;
+  static constexpr int kSumSteps = 16;
+  // per loop position: a draw summed over the loop; a node the loop does not
+  // emit; a node evaluated after it (hoisted, or part of a form the step
+  // reads for something else too)
+  std::vector<char> dsum_, hoist_, after_;
+  void plan_draw_sums();
+  bool linear_form(int pos, double scale, double& offset, std::vector<char>& draws) const;
+  void hoisted_step();
+  std::string body_rhs(int u, int j, const std::string& x, const std::string& y) const;
+  void draw_sum(int U, int u, int j, std::map<std::pair<int, int>, std::string>& pairs,
+                std::set<std::pair<int, int>>& done, const std::string& ind);
   bool gaff(int pos) const { return geo_log(pos) && pos < static_cast<int>(gaff_.size()) && gaff_[pos].on; }
   void geo_affine_finish(int j);
   void l2e_copies();
@@ -1392,6 +1420,16 @@ class Emitter {
                const std::string& Vi, const std::string& Va, const std::string& Vb,
                const std::function<std::string(int)>& ta, const std::function<std::string(int)>& tb);
   void tline(int lo, int hi);
+  void tnode(int lo, int i);
+  void need(int node);
+  void need_l2e(int node);
+  void finish_geo(int j);
+  void finish_carry(int pos);
+  // After the loop: carried positions whose final value is not emitted yet
+  // (empty: not after a loop, or nothing is deferred) and, in a
+  // remat_open scope, set-up nodes and their log2(e) copies likewise.
+  std::vector<char> pending_pos_, pending_geo_, pending_pre_, pending_l2e_;
+  bool remat_ = false;
   void tsegment(int U, const std::string& sg);
   int trip_ = 1;  // loop steps per trip of the pass being emitted
   // Trips start at iteration it_base_ + sg * trip_. A stream that draws an
@@ -2058,34 +2096,82 @@ void Emitter::tangent(const std::string& ind, int op, const std::string& tn, con
 void Emitter::tline(int lo, int hi) {
   pairs_.clear();
   for (int i = lo; i < hi; ++i) {
-    const int op = t_.op[i];
-    if (op == NT_OP_RANDN || op == NT_OP_RANDU) {
-      line_draw(lo, i);  // a draw is never active: one per path, shared by the markets
-      continue;
+    const int ar = is_draw(t_.op[i]) ? 0 : arity(t_.op[i]);
+    if (ar >= 1) need(t_.a[i]);
+    if (ar >= 2) need(t_.b[i]);
+    tnode(lo, i);
+  }
+}
+
+void Emitter::tnode(int lo, int i) {
+  const int op = t_.op[i];
+  if (is_draw(op)) {
+    line_draw(lo, i);  // a draw is never active: one per path, shared by the markets
+    return;
+  }
+  const int ar = arity(op);
+  const bool act = t_.active[i] != 0;
+  for (int m = act ? mlo_ : 0; m < (act ? mhi_ : 1); ++m) {
+    m_ = m;
+    exp_active_ = act;
+    const std::string x = ar >= 1 ? vname(t_.a[i]) : "";
+    const std::string y = ar >= 2 ? vname(t_.b[i]) : "";
+    std::string val = expr(op, x, y, t_.c[i], t_.a[i], i);
+    sqrt_q_.clear();
+    if (op == NT_OP_SQRT && fast_sqrt() && !slow_) {
+      const std::string q = "t" + std::to_string(i) + "_q" + ms(true);
+      o_ << "    real " << q << ";\n";
+      val = sqrt_expr(x, q, act);
     }
-    const int ar = arity(op);
-    const bool act = t_.active[i] != 0;
-    for (int m = act ? mlo_ : 0; m < (act ? mhi_ : 1); ++m) {
-      m_ = m;
-      exp_active_ = act;
-      const std::string x = ar >= 1 ? vname(t_.a[i]) : "";
-      const std::string y = ar >= 2 ? vname(t_.b[i]) : "";
-      std::string val = expr(op, x, y, t_.c[i], t_.a[i], i);
-      sqrt_q_.clear();
-      if (op == NT_OP_SQRT && fast_sqrt() && !slow_) {
-        const std::string q = "t" + std::to_string(i) + "_q" + ms(true);
-        o_ << "    real " << q << ";\n";
-        val = sqrt_expr(x, q, act);
+    recip_ = op == NT_OP_DIV && fast_sqrt() && !slow_ && is_one(t_.a[i]);
+    if (recip_) val = "nt_recip(" + y + ", nt_slow" + ms(act) + ")";
+    o_ << "    const real v" << i << ms(act) << " = " << val << ";\n";
+    if (!act || ar == 0 || !p_.adjoints) continue;
+    const int a = t_.a[i], b = ar >= 2 ? t_.b[i] : -1;
+    tangent("    ", op, "t" + std::to_string(i) + "_", ms(true), deplist(i), "v" + std::to_string(i) + ms(true), x, y,
+            [&](int j) { return tname(a, j); }, [&](int j) { return b >= 0 ? tname(b, j) : std::string(); });
+    sqrt_q_.clear();
+  }
+}
+
+// Where two or more waves per SIMD are asked for (nt_options.waves, or the
+// engine's second compile of a kernel just over two waves' registers), the
+// code after a step loop emits what it reads on first use: a carried value's
+// final form (finish_carry) and, in a scope that computes the set-up values
+// again (remat_open), those values, operands first. Its registers then hold
+// what one asset of a basket needs and the running result, not every asset's
+// set-up and every carry's value with its tangents at once.
+void Emitter::need(int node) {
+  if (pending_pos_.empty() || node < 0) return;
+  if (node >= L_.start && node < L_.end()) {
+    finish_carry(node - (L_.start + (L_.iters - 1) * L_.period));
+    return;
+  }
+  if (node >= static_cast<int>(pending_pre_.size()) || !pending_pre_[node]) return;
+  std::vector<int> stack{node};
+  while (!stack.empty()) {
+    const int i = stack.back();
+    const int ar = is_draw(t_.op[i]) ? 0 : arity(t_.op[i]);
+    bool ready = true;
+    for (int slot = 0; slot < ar; ++slot) {
+      const int x = slot == 0 ? t_.a[i] : t_.b[i];
+      if (pending_pre_[x]) {
+        stack.push_back(x);
+        ready = false;
       }
-      recip_ = op == NT_OP_DIV && fast_sqrt() && !slow_ && is_one(t_.a[i]);
-      if (recip_) val = "nt_recip(" + y + ", nt_slow" + ms(act) + ")";
-      o_ << "    const real v" << i << ms(act) << " = " << val << ";\n";
-      if (!act || ar == 0 || !p_.adjoints) continue;
-      const int a = t_.a[i], b = ar >= 2 ? t_.b[i] : -1;
-      tangent("    ", op, "t" + std::to_string(i) + "_", ms(true), deplist(i), "v" + std::to_string(i) + ms(true), x, y,
-              [&](int j) { return tname(a, j); }, [&](int j) { return b >= 0 ? tname(b, j) : std::string(); });
-      sqrt_q_.clear();
     }
+    if (!ready) continue;
+    stack.pop_back();
+    if (!pending_pre_[i]) continue;
+    pending_pre_[i] = 0;
+    const bool par = par_on_;
+    const int m = m_;
+    par_on_ = false;
+    in_sfx_ = "_r";
+    tnode(0, i);
+    in_sfx_.clear();
+    par_on_ = par;
+    m_ = m;
   }
 }
 
@@ -2123,6 +2209,30 @@ void Emitter::body_tangent_operand(int u, int kind, int ref, std::function<std::
 
 // One trip of U loop iterations: values and their tangents, then the carried
 // state (values and tangents) advances.
+// Value of loop position j in iteration u of the trip, from its operands x
+// and y, for what needs no statement of its own before it.
+std::string Emitter::body_rhs(int u, int j, const std::string& x, const std::string& y) const {
+  const int op = t_.op[L_.start + j];
+  if (!t_.active[L_.start + j] && draw_fma() && (op == NT_OP_ADD || op == NT_OP_SUB)) {
+    const std::string fm = draw_fma_expr(u, j, op);
+    if (!fm.empty()) return fm;
+  }
+  if (op == NT_OP_EXP && fold_[j].on) {
+    const Exp2Fold& f = fold_[j];
+    const std::string sv = body_value(u, f.s_kind, f.s_ref, false);
+    return "nt_hw_exp2f(" + f.arg(f.p >= 0 ? l2e_name(f.p) : "", l2e_name(f.r), sv, p_.fuse) + ")";
+  }
+  if (op == NT_OP_EXP && bound_[j].on && !slow_ && !f32_ && p_.libm != 1) return "nt_exp_core(" + x + ")";
+  if (fused_exp_[j] >= 0 && p_.adjoints) {
+    const ExpBound& b = bound_[fused_exp_[j]];
+    const std::string rv = body_value(u, ARG_INV, b.r, false), pv = body_value(u, ARG_INV, b.p, false);
+    const std::string z = body_value(u, ARG_BODY, b.draw, false);
+    const bool sub = op == NT_OP_SUB;
+    return f("fma") + "(" + (sub && b.p_first ? "-" + rv : rv) + ", " + z + ", " + (sub && !b.p_first ? "-" + pv : pv) + ")";
+  }
+  return body_expr(j, u, op, x, y);
+}
+
 void Emitter::tsegment(int U, const std::string& sg) {
   const int P = L_.period, s = L_.start;
   const std::string ind = "      ";
@@ -2132,16 +2242,21 @@ void Emitter::tsegment(int U, const std::string& sg) {
      << ") * " << trip_ << "u;\n";
   trip_counters(ind);
   std::map<std::pair<int, int>, std::string> pairs;
+  std::set<std::pair<int, int>> summed;  // draws added to their sums with their pair's other leg
   for (int u = 0; u < U; ++u) {
     for (int j = 0; j < P; ++j) {
       const int i = s + j;
       const int op = t_.op[i];
       const std::string name = "r" + std::to_string(u) + "_" + std::to_string(j);
-      if (op == NT_OP_RANDN || op == NT_OP_RANDU) {
-        const std::string d = body_draw(u, j, pairs, ind);
-        o_ << ind << "const real " << name << " = " << d << ";\n";
+      if (is_draw(op)) {
+        if (slow_ || !hoist_[j]) {
+          const std::string d = body_draw(u, j, pairs, ind);
+          o_ << ind << "const real " << name << " = " << d << ";\n";
+        }
+        if (!slow_ && dsum_[j]) draw_sum(U, u, j, pairs, summed, ind);
         continue;
       }
+      if (!slow_ && hoist_[j]) continue;
       const int ar = arity(op);
       const bool act = t_.active[i] != 0;
       if (sched_on_ && !slow_ && sched_[j] && op != NT_OP_CONST) {
@@ -2164,33 +2279,16 @@ void Emitter::tsegment(int U, const std::string& sg) {
         exp_active_ = act;
         const std::string x = ar >= 1 ? body_value(u, L_.kind_a[j], L_.ref_a[j], false) : "";
         const std::string y = ar >= 2 ? body_value(u, L_.kind_b[j], L_.ref_b[j], false) : "";
-        std::string val = body_expr(j, u, op, x, y);
-        if (!act && draw_fma() && (op == NT_OP_ADD || op == NT_OP_SUB)) {
-          const std::string fm = draw_fma_expr(u, j, op);
-          if (!fm.empty()) val = fm;
-        }
-        if (op == NT_OP_EXP && fold_[j].on) {
-          const Exp2Fold& f = fold_[j];
-          const std::string sv = body_value(u, f.s_kind, f.s_ref, false);
-          val = "nt_hw_exp2f(" + f.arg(f.p >= 0 ? l2e_name(f.p) : "", l2e_name(f.r), sv, p_.fuse) + ")";
-        }
+        std::string val = body_rhs(u, j, x, y);
         sqrt_q_.clear();
         if (op == NT_OP_SQRT && fast_sqrt() && !slow_) {
           const std::string q = "tr" + std::to_string(u) + "_" + std::to_string(j) + "_q" + ms(true);
           o_ << ind << "real " << q << ";\n";
           val = sqrt_expr(x, q, act);
         }
-        if (op == NT_OP_EXP && bound_[j].on && !slow_ && !f32_ && p_.libm != 1) val = "nt_exp_core(" + x + ")";
         recip_ = op == NT_OP_DIV && fast_sqrt() && !slow_ &&
                  ((L_.kind_a[j] == ARG_BODY && is_one(s + L_.ref_a[j])) || (L_.kind_a[j] == ARG_INV && is_one(L_.ref_a[j])));
         if (recip_) val = "nt_recip(" + y + ", nt_slow" + ms(act) + ")";
-        if (fused_exp_[j] >= 0 && p_.adjoints) {
-          const ExpBound& b = bound_[fused_exp_[j]];
-          const std::string rv = body_value(u, ARG_INV, b.r, false), pv = body_value(u, ARG_INV, b.p, false);
-          const std::string z = body_value(u, ARG_BODY, b.draw, false);
-          const bool sub = op == NT_OP_SUB;
-          val = f("fma") + "(" + (sub && b.p_first ? "-" + rv : rv) + ", " + z + ", " + (sub && !b.p_first ? "-" + pv : pv) + ")";
-        }
         if (gsum_[j] >= 0 && act && p_.adjoints) {
           // sum of G (the spots' sum is A0 + c0 sum G)
           val = body_value(u, ARG_CARRY, j, false) + " + gq" + std::to_string(u) + "_" + std::to_string(gsum_[j]) + ms(true);
@@ -2205,6 +2303,7 @@ void Emitter::tsegment(int U, const std::string& sg) {
           if (gaff(j)) {
             // the sum of s; exponents and tangents follow after the loop
             const GeoAffine& g = gaff_[j];
+            if (g.linear) continue;
             o_ << ind << "const real zq" << su << "_" << sj << m << " = "
                << (u > 0 ? "zq" + prev + "_" + sj + m : "zs" + sj + m) << " + "
                << body_value(u, g.s_kind, g.s_ref, false) << ";\n";
@@ -2279,6 +2378,7 @@ void Emitter::tsegment(int U, const std::string& sg) {
       if (!(geo_free(j) && act && p_.adjoints)) o_ << ind << "st" << j << sm << " = r" << (U - 1) << "_" << j << sm << ";\n";
       if (!act || !p_.adjoints) continue;
       if (gaff(j)) {
+        if (gaff_[j].linear) continue;
         o_ << ind << "zs" << j << sm << " = zq" << (U - 1) << "_" << j << sm << ";\n";
         continue;
       }
@@ -2500,6 +2600,158 @@ void Emitter::plan_geo_affine() {
     if (g.s_kind != ARG_BODY || t_.active[L_.start + g.s_ref]) continue;
     g.on = true;
     gaff_[j] = g;
+  }
+}
+
+// Whether scale x (the value of loop position pos) is a linear form of the
+// step's draws: marks them in `draws` and adds its constant term to `offset`.
+bool Emitter::linear_form(int pos, double scale, double& offset, std::vector<char>& draws) const {
+  const int op = t_.op[L_.start + pos];
+  if (!std::isfinite(scale)) return false;
+  if (is_draw(op)) {
+    draws[pos] = 1;
+    return true;
+  }
+  if (t_.active[L_.start + pos]) return false;
+  auto literal = [&](int kind, int ref, double& v) {
+    const int node = kind == ARG_BODY ? L_.start + ref : kind == ARG_INV ? ref : -1;
+    if (node < 0 || t_.op[node] != NT_OP_CONST || (kind == ARG_BODY && L_.table_lit(ref))) return false;
+    v = t_.c[node];
+    return true;
+  };
+  auto operand = [&](int kind, int ref, double by) {
+    double v = 0;
+    if (literal(kind, ref, v)) {
+      offset += by * v;
+      return true;
+    }
+    return kind == ARG_BODY && linear_form(ref, by, offset, draws);
+  };
+  const int ka = L_.kind_a[pos], ra = L_.ref_a[pos], kb = L_.kind_b[pos], rb = L_.ref_b[pos];
+  double v = 0;
+  switch (op) {
+    case NT_OP_NEG: return operand(ka, ra, -scale);
+    case NT_OP_ADD: return operand(ka, ra, scale) && operand(kb, rb, scale);
+    case NT_OP_SUB: return operand(ka, ra, scale) && operand(kb, rb, -scale);
+    case NT_OP_MUL:
+      if (literal(kb, rb, v)) return operand(ka, ra, scale * v);
+      return literal(ka, ra, v) && operand(kb, rb, scale * v);
+    case NT_OP_DIV: return literal(kb, rb, v) && operand(ka, ra, scale / v);
+    default: return false;
+  }
+}
+
+void Emitter::plan_draw_sums() {
+  const int P = L_.found ? L_.period : 0;
+  dsum_.assign(P, 0);
+  hoist_.assign(P, 0);
+  after_.assign(P, 0);
+  std::vector<char> sum(P, 0), draws(P, 0);
+  int carries = 0;
+  for (int j = 0; j < P; ++j) {
+    if (!(j < static_cast<int>(gaff_.size()) && gaff_[j].on)) continue;
+    std::vector<char> own(P, 0);
+    double offset = 0;
+    if (!linear_form(gaff_[j].s_ref, 1.0, offset, own) || offset != 0.0) continue;
+    sum[j] = 1;
+    ++carries;
+    for (int d = 0; d < P; ++d) draws[d] |= own[d];
+  }
+  if (!carries) return;
+  // nodes read by nothing but those exponents
+  std::vector<std::vector<int>> users(P);
+  std::vector<char> kept(P, 0), hoist(P, 0);
+  for (int j = 0; j < P; ++j) {
+    kept[j] = L_.is_carry[j] || L_.is_liveout[j];
+    const int ar = is_draw(t_.op[L_.start + j]) ? 0 : arity(t_.op[L_.start + j]);
+    if (ar >= 1 && L_.kind_a[j] == ARG_BODY) users[L_.ref_a[j]].push_back(j);
+    if (ar >= 2 && L_.kind_b[j] == ARG_BODY) users[L_.ref_b[j]].push_back(j);
+  }
+  int saved = carries;
+  for (int j = P - 1; j >= 0; --j) {
+    if (kept[j] || users[j].empty()) continue;
+    hoist[j] = 1;
+    for (int u : users[j]) hoist[j] = hoist[j] && (hoist[u] || sum[u]);
+    const int op = t_.op[L_.start + j];
+    // a product and the sum it feeds are one fma
+    if (hoist[j] && !t_.active[L_.start + j] && (op == NT_OP_ADD || op == NT_OP_SUB)) ++saved;
+  }
+  for (int d = 0; d < P; ++d) saved -= draws[d];
+  if (saved < kSumSaves) return;
+  dsum_ = draws;
+  hoist_ = hoist;
+  after_ = hoist;
+  for (int j = 0; j < P; ++j) {
+    if (!sum[j]) continue;
+    gaff_[j].linear = true;
+    after_[gaff_[j].s_ref] = 1;
+  }
+  for (int j = P - 1; j >= 0; --j) {
+    const int ar = is_draw(t_.op[L_.start + j]) ? 0 : arity(t_.op[L_.start + j]);
+    if (!after_[j]) continue;
+    if (ar >= 1 && L_.kind_a[j] == ARG_BODY) after_[L_.ref_a[j]] = 1;
+    if (ar >= 2 && L_.kind_b[j] == ARG_BODY) after_[L_.ref_b[j]] = 1;
+  }
+}
+
+// Adds draw position j of iteration u (of the U in the trip) to its sum. Both
+// legs of a Box-Muller pair that are read by nothing else go to their sums as
+// radius times leg in one fma each.
+void Emitter::draw_sum(int U, int u, int j, std::map<std::pair<int, int>, std::string>& pairs,
+                       std::set<std::pair<int, int>>& done, const std::string& ind) {
+  const int i = L_.start + j, stream = t_.b[i];
+  const std::string own = "ds" + std::to_string(j);
+  if (t_.op[i] == NT_OP_RANDN && hoist_[j]) {
+    auto sh = draw_shift_.find(stream);
+    const int shift = sh != draw_shift_.end() ? sh->second : 0;
+    const int rel = L_.rand_base[j] + u * L_.rand_step[j] - shift;
+    if (done.count({stream, rel})) return;
+    if (!pairs.count({stream, rel >> 1})) {
+      for (int v = u; v < U; ++v) {
+        for (int k = 0; k < L_.period; ++k) {
+          if (t_.op[L_.start + k] != NT_OP_RANDN || t_.b[L_.start + k] != stream || !hoist_[k] || !dsum_[k]) continue;
+          if (L_.rand_base[k] + v * L_.rand_step[k] - shift != (rel ^ 1)) continue;
+          const std::string other = "ds" + std::to_string(k);
+          o_ << ind << "nt_normal_pair_sum(rlo, " << rhi(stream) << ", (kb" << stream << " >> 1) + " << (rel >> 1)
+             << "u, " << (rel & 1 ? other : own) << ", " << (rel & 1 ? own : other) << ");\n";
+          done.insert({stream, rel ^ 1});
+          return;
+        }
+      }
+    }
+  }
+  const std::string z = hoist_[j] ? body_draw(u, j, pairs, ind) : "r" + std::to_string(u) + "_" + std::to_string(j);
+  o_ << ind << own << " += " << z << ";\n";
+}
+
+// After the loop: the hoisted nodes of a step on the draws' sums, and each
+// carry's S = 0 + s of them.
+void Emitter::hoisted_step() {
+  const std::string ind = "    ";
+  for (int j = 0; j < L_.period; ++j) {
+    const int op = t_.op[L_.start + j];
+    const std::string sj = std::to_string(j);
+    if (dsum_[j]) o_ << ind << "const real r0_" << sj << " = " << (f32_ ? "(real)dds" : "ds") << sj << ";\n";
+    if (!after_[j] || is_draw(op)) continue;
+    const int ar = arity(op);
+    const bool act = t_.active[L_.start + j] != 0;
+    for (int m = act ? mlo_ : 0; m < (act ? mhi_ : 1); ++m) {
+      m_ = m;
+      exp_active_ = act;
+      const std::string x = ar >= 1 ? body_value(0, L_.kind_a[j], L_.ref_a[j], false) : "";
+      const std::string y = ar >= 2 ? body_value(0, L_.kind_b[j], L_.ref_b[j], false) : "";
+      o_ << ind << "const real r0_" << sj << ms(act) << " = " << body_rhs(0, j, x, y) << ";\n";
+    }
+  }
+  for (int j = 0; j < L_.period; ++j) {
+    if (!gaff(j) || !gaff_[j].linear) continue;
+    for (int m = mlo_; m < mhi_; ++m) {
+      m_ = m;
+      const std::string sj = std::to_string(j) + ms(true);
+      o_ << ind << "const real zq0_" << sj << " = zs" << sj << " + "
+         << body_value(0, gaff_[j].s_kind, gaff_[j].s_ref, false) << ";\n";
+      o_ << ind << "zs" << sj << " = zq0_" << sj << ";\n";
+    }
   }
 }
 
@@ -3025,6 +3277,11 @@ void Emitter::body_tangent() {
         }
       }
     }
+    for (int j = 0; j < L_.period && !slow_; ++j) {
+      if (!dsum_[j]) continue;
+      o_ << "    real ds" << j << " = " << zero << ";\n";
+      if (f32_) o_ << "    double dds" << j << " = 0.0;\n";
+    }
     exp_bound_checks();
     // The re-evaluation pass, which runs for a rare path, takes the shortest
     // trip (one step, two when a step draws an odd number of normals) so its
@@ -3038,66 +3295,55 @@ void Emitter::body_tangent() {
       for (const auto& kv : L_.normal_step) draw_shift_[kv.first] = kv.second & 1;
     }
     const int nfull = (L_.iters - lead) / trip_, tail = (L_.iters - lead) % trip_;
-    if (nfull > 0) {
+    bool sums = false;
+    for (int j = 0; j < L_.period && !slow_; ++j) sums |= f32_ && dsum_[j];
+    auto flush = [&](const std::string& ind, bool again) {
+      for (int j = 0; j < L_.period; ++j) {
+        if (!dsum_[j]) continue;
+        const std::string d = "ds" + std::to_string(j);
+        o_ << ind << "d" << d << " += (double)" << d << ";" << (again ? " " + d + " = 0.0f;" : "") << "\n";
+      }
+    };
+    if (nfull > 0 && sums) {
+      const int block = std::max(1, kSumSteps / trip_);
+      o_ << "    for (nt_u32 sb = 0; sb < " << nfull << "u; sb += " << block << "u) {\n"
+         << "    const nt_u32 se = sb + " << block << "u < " << nfull << "u ? sb + " << block << "u : " << nfull << "u;\n"
+         << "    for (nt_u32 sg = sb; sg < se; ++sg)\n";
+      tsegment(trip_, "sg");
+      flush("    ", true);
+      o_ << "    }\n";
+    } else if (nfull > 0) {
       o_ << "    for (nt_u32 sg = 0; sg < " << nfull << "u; ++sg)\n";
       tsegment(trip_, "sg");
     }
     if (tail) tsegment(tail, std::to_string(nfull) + "u");
+    if (sums) flush("    ", false);
+    if (!slow_) hoisted_step();
     it_base_ = 0;
     draw_shift_.clear();
     for (int j = 0; j < L_.period && !slow_; ++j) remat |= gaff(j);
+    par_on_ = false;
+    pending_pos_.assign(L_.period, 1);
+    pending_geo_.assign(L_.period, 1);
+    remat_ = remat;
     if (remat) remat_open(ls);
-    for (int j = 0; j < L_.period; ++j) {
-      if (!geo(j)) continue;
-      for (int m = mlo_; m < mhi_; ++m) {
-        m_ = m;
-        if (gaff(j)) geo_affine_finish(j);
-        if (geo_log(j)) {
-          const bool a_self = L_.kind_a[j] == ARG_CARRY && L_.ref_a[j] == j;
-          const int e = a_self ? L_.ref_b[j] : L_.ref_a[j];
-          const std::string g = "gs" + std::to_string(j) + ms(true);
-          std::string ex;
-          if (f32_) ex = fold_[e].on ? "nt_hw_exp2f(" + g + ")" : "nt_expf(" + g + ")";
-          else ex = p_.libm == 1 ? "exp(" + g + ")" : "nt_exp_fast(" + g + ", nt_slow" + ms(true) + ")";
-          o_ << "    " << g << " = " << ex << ";\n";
-        }
-        if (geo_free(j)) o_ << "    st" << j << ms(true) << " = c0_" << j << ms(true) << " * gs" << j << ms(true) << ";\n";
-        if (gsum_of_[j] >= 0) {
-          const int a = gsum_of_[j];
-          const int init = L_.carry_init[a];
-          const std::string c = "c0_" + std::to_string(j) + ms(true) + " * st" + std::to_string(a) + ms(true);
-          o_ << "    st" << a << ms(true) << " = " << (init >= 0 ? vname(init) + " + " + c : c) << ";\n";
-        }
-        for (int k : posdeplist(j)) {
-          o_ << "    ts" << j << "_" << k << ms(true) << " = gs" << j << ms(true) << " * ts" << j << "_" << k << ms(true)
-             << ";\n";
-        }
-      }
-    }
-    if (par_on_) {
-      // back to the inputs: t_k = sum over parameters d of t_d x (d's tangent for input k)
-      par_on_ = false;
-      const int nin = t_.n_in;
+    if (p_.waves < 2) {
+      // Every set-up value and every final value at once: more of them in
+      // flight, more registers.
+      for (int i = 0; remat && i < ls; ++i) need(i);
       for (int j = 0; j < L_.period; ++j) {
-        if (!(L_.is_carry[j] || L_.is_liveout[j]) || !t_.active[L_.start + j]) continue;
-        for (int m = mlo_; m < mhi_; ++m) {
-          m_ = m;
-          for (int k : posdeplist(j)) {
-            std::string e;
-            for (size_t d = 0; d < par_node_.size(); ++d) {
-              if (!par_deps_[j][d]) continue;
-              const std::string T = tname(par_node_[d], k);
-              if (T.empty()) continue;
-              const std::string td = "ts" + std::to_string(j) + "_" + std::to_string(nin + static_cast<int>(d)) + ms(true);
-              if (T == "#1") e = e.empty() ? td : "(" + e + " + " + td + ")";
-              else e = e.empty() ? "(" + td + " * " + T + ")" : f("fma") + "(" + td + ", " + T + ", " + e + ")";
-            }
-            o_ << "    const " << treal() << " ts" << j << "_" << k << ms(true) << " = " << (e.empty() ? zero : e) << ";\n";
-          }
-        }
+        if (geo(j)) finish_geo(j);
+      }
+      for (int j = 0; j < L_.period; ++j) {
+        if (L_.is_carry[j] || L_.is_liveout[j]) finish_carry(j);
       }
     }
     tline(le, n);
+    for (int out : t_.outputs) need(out);
+    pending_pos_.clear();
+    pending_geo_.clear();
+    pending_pre_.clear();
+    pending_l2e_.clear();
   }
   const int nin = t_.n_in;
   for (int m = mlo_; m < mhi_; ++m) {
@@ -3116,59 +3362,138 @@ void Emitter::body_tangent() {
   if (remat) o_ << "    }\n";
 }
 
-// fp32 exp2 folds: p log2(e) and r log2(e) of every folded exponent
-void Emitter::l2e_copies() {
-  std::set<int> scaled;
-  for (const auto& f : fold_) {
-    if (!f.on) continue;
-    if (f.p >= 0) scaled.insert(f.p);
-    scaled.insert(f.r);
-  }
-  for (int node : scaled) {
-    const bool act = t_.active[node] != 0;
-    for (int m = act ? mlo_ : 0; m < (act ? mhi_ : 1); ++m) {
-      m_ = m;
-      o_ << "    const real " << l2e_name(node) << " = " << vname(node) << " * 1.44269504088896341f;\n";
-    }
-  }
-}
-
-// After the step loop: a scope that computes the values before the loop
-// again, from opaque copies of the inputs, so the code after the loop reads
-// these copies and the compiler keeps nothing of the path's set-up live
-// through the loop but what the loop itself reads. The inputs are uniform, so
-// the copies stay in SGPRs; the set-up is a few hundred operations per path,
-// against the loop's hundreds per step.
-void Emitter::remat_open(int ls) {
+// After the loop: geo carry j's value and tangents in absolute form.
+void Emitter::finish_geo(int j) {
+  if (!pending_geo_[j]) return;
+  pending_geo_[j] = 0;
   const std::string zero = f32_ ? "0.0f" : "0.0";
   const std::string one = f32_ ? "1.0f" : "1.0";
+  const int init = L_.carry_init[j];
+  if (remat_) need(init);
+  if (gaff(j)) {
+    const GeoAffine& g = gaff_[j];
+    need(g.p);
+    need(g.r);
+    if (f32_) {
+      if (g.p >= 0) need_l2e(g.p);
+      need_l2e(g.r);
+    }
+  }
+  par_on_ = use_par_;
+  for (int m = mlo_; m < mhi_; ++m) {
+    m_ = m;
+    if (remat_) {
+      o_ << "    const real c0_" << j << ms(true) << " = " << (init >= 0 ? vname(init) : zero) << ";\n";
+      // the loop leaves these tangents at their start values
+      for (int k : posdeplist(j)) {
+        if (!gaff(j)) break;
+        const std::string tin = init >= 0 ? inv_tname(init, k) : "";
+        o_ << "    ts" << j << "_" << k << ms(true) << " = " << (tin.empty() ? zero : tin == "#1" ? one : tin) << ";\n";
+      }
+    }
+    if (gaff(j)) geo_affine_finish(j);
+    if (geo_log(j)) {
+      const bool a_self = L_.kind_a[j] == ARG_CARRY && L_.ref_a[j] == j;
+      const int e = a_self ? L_.ref_b[j] : L_.ref_a[j];
+      const std::string g = "gs" + std::to_string(j) + ms(true);
+      std::string ex;
+      if (f32_) ex = fold_[e].on ? "nt_hw_exp2f(" + g + ")" : "nt_expf(" + g + ")";
+      else ex = p_.libm == 1 ? "exp(" + g + ")" : "nt_exp_fast(" + g + ", nt_slow" + ms(true) + ")";
+      o_ << "    " << g << " = " << ex << ";\n";
+    }
+    if (geo_free(j)) o_ << "    st" << j << ms(true) << " = c0_" << j << ms(true) << " * gs" << j << ms(true) << ";\n";
+    if (gsum_of_[j] >= 0) {
+      const int a = gsum_of_[j];
+      const int ia = L_.carry_init[a];
+      if (remat_) need(ia);
+      const std::string c = "c0_" + std::to_string(j) + ms(true) + " * st" + std::to_string(a) + ms(true);
+      o_ << "    st" << a << ms(true) << " = " << (ia >= 0 ? vname(ia) + " + " + c : c) << ";\n";
+    }
+    for (int k : posdeplist(j)) {
+      o_ << "    ts" << j << "_" << k << ms(true) << " = gs" << j << ms(true) << " * ts" << j << "_" << k << ms(true)
+         << ";\n";
+    }
+  }
+  par_on_ = false;
+}
+
+// After the loop: the final value of carried (or live-out) position pos, its
+// tangents back over the inputs where the loop ran over parameters: t_k = sum
+// over parameters d of t_d x (d's tangent for input k).
+void Emitter::finish_carry(int pos) {
+  if (pos < 0 || !pending_pos_[pos]) return;
+  pending_pos_[pos] = 0;
+  const int m0 = m_;
+  if (geo(pos)) finish_geo(pos);
+  if (gsum_[pos] >= 0) finish_geo(gsum_[pos]);
+  if (use_par_ && t_.active[L_.start + pos]) {
+    const std::string zero = f32_ ? "0.0f" : "0.0";
+    const int nin = t_.n_in;
+    for (size_t d = 0; remat_ && d < par_node_.size(); ++d) {
+      if (par_deps_[pos][d]) need(par_node_[d]);
+    }
+    for (int m = mlo_; m < mhi_; ++m) {
+      m_ = m;
+      for (int k : posdeplist(pos)) {
+        std::string e;
+        for (size_t d = 0; d < par_node_.size(); ++d) {
+          if (!par_deps_[pos][d]) continue;
+          const std::string T = tname(par_node_[d], k);
+          if (T.empty()) continue;
+          const std::string td = "ts" + std::to_string(pos) + "_" + std::to_string(nin + static_cast<int>(d)) + ms(true);
+          if (T == "#1") e = e.empty() ? td : "(" + e + " + " + td + ")";
+          else e = e.empty() ? "(" + td + " * " + T + ")" : f("fma") + "(" + td + ", " + T + ", " + e + ")";
+        }
+        o_ << "    const " << treal() << " ts" << pos << "_" << k << ms(true) << " = " << (e.empty() ? zero : e) << ";\n";
+      }
+    }
+  }
+  m_ = m0;
+}
+
+// fp32 exp2 folds: p log2(e) and r log2(e) of every folded exponent
+void Emitter::l2e_copies() {
+  pending_l2e_.assign(t_.n, 0);
+  for (const auto& f : fold_) {
+    if (!f.on) continue;
+    if (f.p >= 0) pending_l2e_[f.p] = 1;
+    pending_l2e_[f.r] = 1;
+  }
+  for (int node = 0; node < t_.n; ++node) need_l2e(node);
+}
+
+void Emitter::need_l2e(int node) {
+  if (node >= static_cast<int>(pending_l2e_.size()) || !pending_l2e_[node]) return;
+  pending_l2e_[node] = 0;
+  const bool act = t_.active[node] != 0;
+  const int m0 = m_;
+  for (int m = act ? mlo_ : 0; m < (act ? mhi_ : 1); ++m) {
+    m_ = m;
+    o_ << "    const real " << l2e_name(node) << " = " << vname(node) << " * 1.44269504088896341f;\n";
+  }
+  m_ = m0;
+}
+
+// After the step loop: a scope in which the values before the loop are
+// computed again (need), from opaque copies of the inputs, so the code after
+// the loop reads these copies and the compiler keeps nothing of the path's
+// set-up live through the loop but what the loop itself reads. The inputs are
+// uniform, so the copies stay in SGPRs; the set-up is a few hundred operations
+// per path, against the loop's hundreds per step.
+void Emitter::remat_open(int ls) {
   o_ << "    {\n";
   for (int m = mlo_; m < mhi_; ++m) {
     for (int j = 0; j < t_.n_in; ++j) {
       o_ << "    const real in" << j << msuf(m) << "_r = nt_opaque_u(in" << j << msuf(m) << ");\n";
     }
   }
-  const bool par = par_on_;
-  par_on_ = false;
   scal_.clear();
-  in_sfx_ = "_r";
-  tline(0, ls);
-  in_sfx_.clear();
-  l2e_copies();
-  par_on_ = par;
-  for (int j = 0; j < L_.period; ++j) {
-    if (!geo(j) || !t_.active[L_.start + j] || !p_.adjoints) continue;
-    const int init = L_.carry_init[j];
-    for (int m = mlo_; m < mhi_; ++m) {
-      m_ = m;
-      o_ << "    const real c0_" << j << ms(true) << " = " << (init >= 0 ? vname(init) : zero) << ";\n";
-      if (!gaff(j)) continue;
-      // the loop leaves these tangents at their start values
-      for (int k : posdeplist(j)) {
-        const std::string tin = init >= 0 ? inv_tname(init, k) : "";
-        o_ << "    ts" << j << "_" << k << ms(true) << " = " << (tin.empty() ? zero : tin == "#1" ? one : tin) << ";\n";
-      }
-    }
+  pending_pre_.assign(ls, 1);
+  pending_l2e_.assign(t_.n, 0);
+  for (const auto& f : fold_) {
+    if (!f.on) continue;
+    if (f.p >= 0) pending_l2e_[f.p] = 1;
+    pending_l2e_[f.r] = 1;
   }
 }
 
@@ -3365,6 +3690,7 @@ std::string Emitter::run() {
   plan_geo_logs();
   plan_fused_exponents();
   plan_geo_affine();
+  plan_draw_sums();
   par_on_ = false;
   preamble();
   kernel(false);

@@ -359,47 +359,66 @@ __device__ __forceinline__ float nt_uniformf(nt_u32 lo, nt_u32 hi, nt_u32 k) {
   return static_cast<float>(nt_uniform(lo, hi, k));
 }
 
-// Both legs of the Box-Muller pair for Philox counter `ctr` of a path whose
-// counter words are (lo, hi): u = (c + 0.5) * 2^-32, r = sqrt(-2 log u1),
-// z = r cos(2 pi u2) for even draws and r sin(2 pi u2) for odd ones. With
-// NT_DEVICE_LIBM the reference expression is evaluated with device libm.
-__device__ __forceinline__ void nt_normal_pair(nt_u32 lo, nt_u32 hi, nt_u32 ctr, double& zc, double& zs) {
+// The Box-Muller pair for Philox counter `ctr` of a path whose counter words
+// are (lo, hi): u = (c + 0.5) * 2^-32, radius r = sqrt(-2 log u1) and the legs
+// cos and sin of 2 pi u2, the draws being r cos for even ordinals and r sin for
+// odd ones. With NT_DEVICE_LIBM the reference expression is evaluated with
+// device libm.
+__device__ __forceinline__ void nt_normal_polar(nt_u32 lo, nt_u32 hi, nt_u32 ctr, double& r, double& c, double& s) {
   nt_u32 c0, c1;
   nt_philox(lo, hi ^ ctr, c0, c1);
 #ifdef NT_DEVICE_LIBM
   const double u1 = (static_cast<double>(c0) + 0.5) * NT_UINT_SCALE;
   const double u2 = (static_cast<double>(c1) + 0.5) * NT_UINT_SCALE;
-  const double r = sqrt(-2.0 * log(u1));
+  r = sqrt(-2.0 * log(u1));
   const double theta = 6.283185307179586 * u2;
-  double s, c;
   sincos(theta, &s, &c);
 #elif defined(NT_LIBM_SINCOS)
-  const double r = nt_sqrt_pos(nt_neg2log_u32(c0));
+  r = nt_sqrt_pos(nt_neg2log_u32(c0));
   const double u2 = (static_cast<double>(c1) + 0.5) * NT_UINT_SCALE;
-  double s, c;
   sincos(6.283185307179586 * u2, &s, &c);
 #else
-  const double r = nt_sqrt_pos(nt_neg2log_u32(c0));
-  double s, c;
+  r = nt_sqrt_pos(nt_neg2log_u32(c0));
   nt_sincos_2pi_u32(c1, s, c);
 #endif
-  zc = r * c;
-  zs = r * s;
 }
 
-// fp32 pair: same counters and the reference's fp32 u; the transcendentals
-// are the hardware ones: ln u1 = ln2 * log2(u1), and sin/cos of 2 pi u2 read
-// u2 directly as revolutions (no multiplication by 2 pi rounds the angle).
-__device__ __forceinline__ void nt_normal_pair(nt_u32 lo, nt_u32 hi, nt_u32 ctr, float& zc, float& zs) {
+// fp32: same counters and the reference's fp32 u; the transcendentals are the
+// hardware ones: ln u1 = ln2 * log2(u1), and sin/cos of 2 pi u2 read u2
+// directly as revolutions (no multiplication by 2 pi rounds the angle).
+__device__ __forceinline__ void nt_normal_polar(nt_u32 lo, nt_u32 hi, nt_u32 ctr, float& r, float& c, float& s) {
   nt_u32 c0, c1;
   nt_philox(lo, hi ^ ctr, c0, c1);
   // (float(c) + 0.5f) * 2^-32 in one rounding: the same float for every c
   // (exact below 2^24; above, both round the same tie or sub-half-ulp term).
   const float u1 = fmaf(static_cast<float>(c0), 0x1p-32f, 0x1p-33f);
   const float u2 = fmaf(static_cast<float>(c1), 0x1p-32f, 0x1p-33f);
-  const float r = nt_hw_sqrtf(-1.38629436111989061f * nt_hw_log2f(u1));  // -2 ln 2 * log2(u1)
-  zc = r * nt_hw_cos2pif(u2);
-  zs = r * nt_hw_sin2pif(u2);
+  r = nt_hw_sqrtf(-1.38629436111989061f * nt_hw_log2f(u1));  // -2 ln 2 * log2(u1)
+  c = nt_hw_cos2pif(u2);
+  s = nt_hw_sin2pif(u2);
+}
+
+// Both draws of a pair.
+template <typename T>
+__device__ __forceinline__ void nt_normal_pair(nt_u32 lo, nt_u32 hi, nt_u32 ctr, T& zc, T& zs) {
+  T r, c, s;
+  nt_normal_polar(lo, hi, ctr, r, c, s);
+  zc = r * c;
+  zs = r * s;
+}
+
+// Adds both draws of a pair to running sums (which may be the same one).
+__device__ __forceinline__ void nt_normal_pair_sum(nt_u32 lo, nt_u32 hi, nt_u32 ctr, double& sumc, double& sums) {
+  double r, c, s;
+  nt_normal_polar(lo, hi, ctr, r, c, s);
+  sumc = fma(r, c, sumc);
+  sums = fma(r, s, sums);
+}
+__device__ __forceinline__ void nt_normal_pair_sum(nt_u32 lo, nt_u32 hi, nt_u32 ctr, float& sumc, float& sums) {
+  float r, c, s;
+  nt_normal_polar(lo, hi, ctr, r, c, s);
+  sumc = fmaf(r, c, sumc);
+  sums = fmaf(r, s, sums);
 }
 
 #ifndef NT_HOST_EMU  // the lowering's CPU tests provide their own reductions

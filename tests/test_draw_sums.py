@@ -1,0 +1,95 @@
+"""A step's linear map of its draws, taken once on the draws' sums after the
+loop: baskets of GBM spots read only by the payoff, whose step exponents take
+correlated normals (rows of a literal matrix), compiled for the host and held
+to the oracle per path. Cases: three to five assets (three is the smallest
+basket that takes it), an odd number of draws per step (Box-Muller pairs split
+over two steps), step counts around the fp32 sums' 16 steps, rows written as
+differences, a draw that the step also reads by
+itself, a row that another value of the step reads, uniforms among the draws,
+and several markets."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import emu
+import oracle
+from conftest import check_per_path, rel_err, tape_slots
+
+OFFSET = 0x100000003
+
+
+def basket(nt, assets, draws, steps, form):
+    """max(sum of the spots - K, 0); asset i's normal is row i of a literal
+    matrix times the step's draws, in the shape `form` names."""
+    dt = 1.0 / steps
+    g = np.random.Generator(np.random.PCG64(assets * 100 + draws))
+    a = g.uniform(-0.6, 0.6, (assets, draws))
+
+    def body(rec):
+        spots = [rec.input(f"S{i}", 90.0 + 5.0 * i) for i in range(assets)]
+        vols = [rec.input(f"v{i}", 0.15 + 0.05 * i) for i in range(assets)]
+        rate = rec.input("r", 0.03)
+        p = [rate.sub(v.mul(v).mul(0.5)).mul(dt) for v in vols]
+        r = [v.mul(dt ** 0.5) for v in vols]
+        state = list(spots)
+        extra = rec.constant(0.0)
+        for _ in range(steps):
+            z = [rec.randu() if form == "uniform" and d == 0 else rec.randn() for d in range(draws)]
+            rows = []
+            for i in range(assets):
+                w = rec.constant(0.0)
+                for d in range(draws):
+                    if form == "signed" and d % 2:
+                        w = w.sub(z[d].mul(-a[i, d]))
+                    else:
+                        w = w.add(z[d].mul(a[i, d]))
+                rows.append(w)
+            if form == "draw_read":
+                extra = extra.add(z[0].mul(rate))
+            if form == "row_read":
+                extra = extra.add(rows[1].mul(rate))
+            for i in range(assets):
+                state[i] = state[i].mul(p[i].add(r[i].mul(rows[i])).exp())
+        total = extra
+        for s in state:
+            total = total.add(s)
+        rec.output(total.sub(90.0 * assets).max(rec.constant(0.0)))
+    return nt.AadRecorder.record(body).flat()
+
+
+CASES = [(3, 3, 16, "rows"), (3, 4, 17, "rows"), (4, 4, 15, "signed"), (5, 3, 40, "signed"), (4, 4, 33, "draw_read"),
+         (4, 4, 20, "row_read"), (4, 3, 31, "uniform"), (5, 5, 48, "rows")]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("assets,draws,steps,form", CASES)
+def test_draw_sums_match_the_oracle(nt, assets, draws, steps, form, precision):
+    from nablatensor_amd import rocm
+    flat = basket(nt, assets, draws, steps, form)
+    src = rocm.lower(flat, rocm.options(precision, mode=2))
+    fast = src[:src.index("nt_replay_slow")]
+    assert "real ds" in fast and "real ds" not in src[len(fast):]
+    k = emu.EmulatedKernel(src, len(flat["input_node"]), tape_slots(src))
+    _, v, g = k.run(flat["recorded_inputs"], 150, OFFSET, 42, grid=2, block=64)
+    if precision == "fp64":
+        check_per_path(v, g, flat, 150, OFFSET, 42, min_strict=0.9)
+    else:
+        # fp32 rounding of the draws (2^-24 |z| each) through 48 steps at most, on spots of about 100
+        ov, og = oracle.replay_paths(flat, 150, OFFSET, 42, f32=True, threads=1)
+        assert rel_err(v, ov) < 2e-4 and rel_err(g, og) < 2e-3
+
+
+def test_draw_sums_shared_by_the_markets(nt):
+    """Several markets share the sums of the draws and keep the single kernel's bits."""
+    from nablatensor_amd import rocm
+    flat = basket(nt, 4, 4, 20, "rows")
+    x0 = np.array(flat["recorded_inputs"])
+    sets = np.stack([x0, x0 * 1.02, x0 * 0.97])
+    src = rocm.lower(flat, rocm.options("fp64", markets=3))
+    assert src[:src.index("nt_replay_slow")].count("real ds0 =") == 1
+    sums, v, g = emu.EmulatedKernel(src, len(x0), 0).run(sets, 120, OFFSET, 7, grid=2, block=64, markets=3)
+    one = rocm.lower(flat, rocm.options("fp64", mode=2))
+    for m in range(3):
+        s1, v1, g1 = emu.EmulatedKernel(one, len(x0), 0).run(sets[m], 120, OFFSET, 7, grid=2, block=64)
+        assert np.array_equal(v[m], v1) and np.array_equal(g[m], g1) and np.array_equal(sums[m], s1)
