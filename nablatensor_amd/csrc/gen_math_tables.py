@@ -1,24 +1,26 @@
 """Generates nt_math_tables.h: constants of the skeleton's own fp64 math.
 
 * log (Tang's table-driven method, ACM TOMS 16(4), 1990), producing -2 ln u
-  for Box-Muller: for the reduced argument x in [sqrt(1/2), sqrt(2)), F is x
-  rounded to 8 fractional bits of its binade; the table holds -2/F and
-  -2 ln(F) as head + tail (heads on a 2^-42 grid, -2 ln 2's head with 42
-  bits, so e (-2 ln2_hi) + head is exact), indexed by (bits(F).hi -
-  0x3FE6A000) >> 12 (257 entries; F = 1 sits at index 150). ln(1 + r),
-  |r| <= 2^-9, is the Taylor polynomial through r^6 (truncation below
-  r^6/7 < 1e-17 relative), rewritten in r' = -2 r.
+  for Box-Muller: the argument is scaled to x in about [3/4, 3/2) and F is x
+  rounded to 8 fractional bits of its binade, F = from_hi(0x3FE80000 + (j <<
+  12)), j = 0..255 (F = 1 at j = 128). The table holds i' = -2 i with i the
+  double nearest 1/F, so that r' = -2 (x i - 1) is one fma, exact to a
+  rounding, and 2 ln i as head + tail (heads on a 2^-42 grid, -2 ln 2's head
+  with 42 bits, so e (-2 ln2_hi) + head is exact). ln(1 + r), |r| <= 2^-9, is
+  the Taylor polynomial through r^6 (truncation below r^6/7 < 1e-17 relative),
+  rewritten in r' = -2 r.
 * exp (Tang's table-driven method, ACM TOMS 15(2), 1989): x = (256 m + j)
-  ln2/256 + r, |r| <= ln2/512; the table holds 2^(j/256) as head + tail,
-  interleaved (t[2j], t[2j+1]) so one LDS read fetches both; ln2/256 is split
-  into a head with 32 significant bits and a tail; exp(r) - 1 is the Taylor
-  polynomial through r^4.
-* sin / cos of 2 pi u on the full circle: u = j/512 + f, |f| <= 2^-10 turns,
-  the table holds (sin, cos)(2 pi j / 512) interleaved; sin(2 pi f) is odd
-  through f^5 (Taylor in f, coefficients (2 pi)^k / k!; truncation below
-  2e-17 relative) and cos(2 pi f) - 1 through f^4 (Taylor, with the f^4
-  coefficient moved to level the error on |f| <= 2^-10: below 8e-18).
-* ln 2 as a double-double; the reference's 2 pi literal and its error.
+  ln2/256 + r, |r| <= ln2/512; the table holds 2^(j/256) as head and tail;
+  ln2/256 is split into a head with 32 significant bits and a tail; exp(r) - 1
+  is the Taylor polynomial through r^4.
+* sin / cos on the full circle: the angle's sector j (of 512) has a table
+  angle a_j near its middle, a multiple of 2^-40 chosen so that sin a_j and cos
+  a_j are doubles to within a few hundredths of an ulp (accurate tables: Gal
+  and Bachelis, ACM TOMS 17(1), 1991), and those two; w = theta - a_j, |w| <=
+  pi/512 + 2^-28, sin w through w^5 (Taylor, truncation below
+  7e-20) and cos w - 1 through w^4 (Taylor, with the w^4 coefficient moved to
+  level the error: below 1e-17).
+* ln 2 as a double-double; the reference's 2 pi literal.
 All values are computed here with mpmath at 60 digits and rounded once.
 Run: python nablatensor_amd/csrc/gen_math_tables.py
 """
@@ -28,6 +30,7 @@ import struct
 from pathlib import Path
 
 import mpmath as mp
+import numpy as np
 
 mp.mp.dps = 60
 
@@ -54,14 +57,15 @@ def main() -> None:
     # Every log entry is stored times -2 (exact), so the kernel gets -2 ln u
     # without a final multiply: the same bits as -2 * (Tang's ln u).
     inv, lo_hi, lo_lo = [], [], []
-    for idx in range(257):
-        F = from_hi(0x3FE6A000 + (idx << 12))
-        inv.append(-2.0 * float(mp.mpf(1) / mp.mpf(F)))
-        l = mp.log(mp.mpf(F))
+    for idx in range(256):
+        F = from_hi(0x3FE80000 + (idx << 12))
+        i = float(mp.mpf(1) / mp.mpf(F))
+        inv.append(-2.0 * i)
+        l = -mp.log(mp.mpf(i))
         h = head(l, -43)
         lo_hi.append(-2.0 * h)
         lo_lo.append(-2.0 * float(l - mp.mpf(h)))
-    assert from_hi(0x3FE6A000 + (150 << 12)) == 1.0 and lo_hi[150] == 0.0
+    assert inv[128] == -2.0 and lo_hi[128] == 0.0 and lo_lo[128] == 0.0
     ln2 = mp.log(2)
     ln2_hi = head(ln2, -42)
     ln2_lo = float(ln2 - mp.mpf(ln2_hi))
@@ -77,7 +81,7 @@ def main() -> None:
     tp = 2 * mp.pi
     two_pi_d = 6.283185307179586  # the reference's literal for 2 pi (Philox.java:74)
     lines.append(f"#define NT_TWO_PI_D {hexd(two_pi_d)}")
-    lines.append(f"#define NT_TWO_PI_D_ERR {hexd(float(mp.mpf(two_pi_d) - tp))}  /* NT_TWO_PI_D - 2 pi */")
+    lines.append(f"#define NT_TWO_PI_U32 {hexd(two_pi_d * 2.0 ** -32)}  /* NT_TWO_PI_D 2^-32, exact */")
     # exp: 2^(j/256) head + tail, ln2/256 = L_hi (32 significant bits) + L_lo
     l64 = ln2 / 256
     e = mp.floor(mp.log(l64, 2))
@@ -89,48 +93,59 @@ def main() -> None:
     lines.append(f"#define NT_EXP_L_LO {hexd(l_lo)}")
     for k in range(2, 5):
         lines.append(f"#define NT_EXP_C{k} {hexd(float(mp.mpf(1) / mp.factorial(k)))}")
-    exp_t = []
+    exp_h, exp_l = [], []
     for j in range(256):
         v = mp.mpf(2) ** (mp.mpf(j) / 256)
         h = float(v)
-        exp_t += [h, float(v - mp.mpf(h))]
-    lines.append("")
-    lines.append("struct NtExpTable {\n  double t[512];  /* t[2j] + t[2j+1] = 2^(j/256) */\n};")
-    lines.append("#define NT_EXP_TABLE_INIT { { \\")
-    lines.append("  " + arr(exp_t).replace("\n", " \\\n") + " } }")
-    # sin/cos of 2 pi f in turns: odd polynomial through f^5, cos - 1 through f^4
-    for k in (1, 3, 5):
-        lines.append(f"#define NT_SC_S{k} {hexd(float((-1) ** (k // 2) * tp ** k / mp.factorial(k)))}")
-    # cos(2 pi f) - 1 = t (C2 + C4 t), t = f^2 <= T = 2^-20: C4 also takes the
-    # f^6 term's share that minimises the largest error on [0, T]. The error
-    # left is t^2 (delta - c6 t) with delta = C4' - C4 and c6 the f^6 Taylor
-    # coefficient; delta = beta c6 T with 4 beta^3 / 27 = 1 - beta levels the
-    # interior extremum (at t = 2 beta T / 3) with the end point t = T, a
-    # tenth of the plain truncation c6 T^3.
-    c6 = -(tp ** 6) / mp.factorial(6)
-    beta = mp.findroot(lambda b: 4 * b ** 3 / 27 - (1 - b), 0.9)
-    cos_c = {2: -(tp ** 2) / 2, 4: tp ** 4 / 24 + beta * c6 * mp.mpf(2) ** -20}
-    for k in (2, 4):
-        lines.append(f"#define NT_SC_C{k} {hexd(float(cos_c[k]))}")
-    sc_t = []
-    for j in range(512):
-        a = tp * j / 512
-        sc_t += [float(mp.sin(a)), float(mp.cos(a))]
-    lines.append("")
-    lines.append("struct NtSinCosTable {\n  double t[1024];  /* t[2j], t[2j+1] = sin, cos of 2 pi j / 512 */\n};")
-    lines.append("#define NT_SINCOS_TABLE_INIT { { \\")
-    lines.append("  " + arr(sc_t).replace("\n", " \\\n") + " } }")
-    lines.append("")
-    lines.append("struct NtLogTable {\n  double inv[257];  /* -2 / F */\n  double hi[257];  /* -2 ln F, head */\n"
-                 "  double lo[257];  /* -2 ln F, tail */\n};")
+        exp_h.append(h)
+        exp_l.append(float(v - mp.mpf(h)))
 
-    lines.append("#define NT_LOG_TABLE_INIT { \\")
-    lines.append("  {" + arr(inv).replace("\n", " \\\n") + "}, \\")
-    lines.append("  {" + arr(lo_hi).replace("\n", " \\\n") + "}, \\")
-    lines.append("  {" + arr(lo_lo).replace("\n", " \\\n") + "} }")
+    def struct(name, init, fields):
+        lines.append("")
+        lines.append("struct __attribute__((aligned(16))) " + name + " {")
+        for f, vals, note in fields:
+            pad = 1 if len(fields) > 1 else 0
+            lines.append(f"  double {f}[{len(vals) + pad}];  /* {note} */")
+        lines.append("};")
+        lines.append(f"#define {init} {{ \\")
+        lines.append(", \\\n".join("  {" + arr(vals).replace("\n", " \\\n") + "}" for _, vals, _ in fields) + " }")
+
+    def pairs(a, b):
+        return [v for ab in zip(a, b) for v in ab]
+
+    struct("NtExpTable", "NT_EXP_TABLE_INIT", [("t", pairs(exp_h, exp_l), "t[2j] + t[2j+1] = 2^(j/256)")])
+    # sin w = w + w t (S3 + S5 t), cos w - 1 = t (-1/2 + C4 t), t = w^2
+    for k in (3, 5):
+        lines.append(f"#define NT_SC_S{k} {hexd(float(mp.mpf((-1) ** (k // 2)) / mp.factorial(k)))}")
+    # t <= T = (pi/512)^2: C4 also takes the w^6 term's share that minimises
+    # the largest error on [0, T]. The error left is t^2 (delta - c6 t) with
+    # delta = C4' - C4 and c6 the w^6 Taylor coefficient; delta = beta c6 T
+    # with 4 beta^3 / 27 = 1 - beta levels the interior extremum (at t = 2
+    # beta T / 3) with the end point t = T, a tenth of the plain truncation.
+    c6 = -mp.mpf(1) / mp.factorial(6)
+    beta = mp.findroot(lambda b: 4 * b ** 3 / 27 - (1 - b), 0.9)
+    lines.append(f"#define NT_SC_C4 {hexd(float(mp.mpf(1) / 24 + beta * c6 * (mp.pi / 512) ** 2))}")
+    ang, sn, cs = [], [], []
+    for j in range(512):
+        a = float(mp.nint(tp * (j + mp.mpf(1) / 2) / 512 * 2 ** 40) / mp.mpf(2) ** 40)
+        # of the 8,193 multiples of 2^-40 around it, the angle whose sine and
+        # cosine both lie closest to doubles (searched in long double)
+        near = (a + np.arange(-4096, 4097) * 2.0 ** -40).astype(np.longdouble)
+        off = np.maximum(*(np.abs(v - v.astype(np.float64)) / np.spacing(np.abs(v.astype(np.float64)))
+                           for v in (np.sin(near), np.cos(near))))
+        a = float(near[np.argmin(off)])
+        ang.append(a)
+        sn.append(float(mp.sin(mp.mpf(a))))
+        cs.append(float(mp.cos(mp.mpf(a))))
+    struct("NtSinCosTable", "NT_SINCOS_TABLE_INIT",
+           [("sin", sn, "sin a_j"), ("cos", cs, "cos a_j"), ("ang", ang, "a_j, near 2 pi (j + 1/2) / 512")])
+    struct("NtLogTable", "NT_LOG_TABLE_INIT",
+           [("inv", inv, "-2 i, i = 1/F rounded"), ("hi", lo_hi, "2 ln i, head"), ("lo", lo_lo, "tail")])
     lines.append("")
-    lines.append("// All tables in one LDS block; 16-byte aligned so each (sin, cos) and")
-    lines.append("// (head, tail) pair is one ds_read_b128 with its offset folded.")
+    lines.append("// All tables in one LDS block. Columns that share an index are arrays of their own")
+    lines.append("// (one address for all of them), one entry longer than they need: at a distance that")
+    lines.append("// is a multiple of 512 bytes two reads become one ds_read2st64_b64, which kept the")
+    lines.append("// LDS busy 3.6 times as long as the two (SQ_LDS_IDX_ACTIVE of the Asian kernel).")
     lines.append("struct __attribute__((aligned(16))) NtTables {\n  NtSinCosTable sc;\n  NtExpTable ex;\n  NtLogTable lg;\n};")
     lines.append("#define NT_TABLES_INIT { NT_SINCOS_TABLE_INIT, NT_EXP_TABLE_INIT, NT_LOG_TABLE_INIT }")
     out = Path(__file__).resolve().parent / "nt_math_tables.h"

@@ -161,13 +161,36 @@ __device__ __forceinline__ float nt_expf(float x) { return nt_hw_exp2f(x * 1.442
 __constant__ NtTables nt_tables_c = NT_TABLES_INIT;
 __shared__ NtTables nt_tables;
 
+struct __attribute__((aligned(16))) NtPair {
+  double a, b;
+};
+
+// Each thread's 16-byte loads of a batch are issued before its first LDS
+// store, so a block waits for about one memory round trip.
 __device__ __forceinline__ void nt_tables_load() {
-  const double* src = reinterpret_cast<const double*>(&nt_tables_c);
-  double* dst = reinterpret_cast<double*>(&nt_tables);
-  constexpr unsigned n = sizeof(NtTables) / sizeof(double);
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+  const NtPair* src = reinterpret_cast<const NtPair*>(&nt_tables_c);
+  NtPair* dst = reinterpret_cast<NtPair*>(&nt_tables);
+  constexpr unsigned n = sizeof(NtTables) / sizeof(NtPair), kBatch = 6;
+  for (unsigned base = threadIdx.x; base < n; base += kBatch * blockDim.x) {
+    double a[kBatch], b[kBatch];
+#pragma unroll
+    for (unsigned k = 0; k < kBatch; ++k) {
+      const unsigned i = base + k * blockDim.x;
+      const NtPair* from = src + (i < n ? i : n - 1);
+      a[k] = from->a;
+      b[k] = from->b;
+    }
+#pragma unroll
+    for (unsigned k = 0; k < kBatch; ++k) {
+      const unsigned i = base + k * blockDim.x;
+      if (i < n) dst[i] = NtPair{a[k], b[k]};
+    }
+  }
   __syncthreads();
 }
+
+// Entry j of a table of pairs, one ds_read_b128.
+__device__ __forceinline__ NtPair nt_pair(const double* t, nt_u32 j) { return reinterpret_cast<const NtPair*>(t)[j]; }
 
 // exp(x) by Tang's table-driven method: x = (256 m + j) ln2/256 + r with
 // |r| <= ln2/512 (ln2/256 split in a 32-bit head and a tail, so the reduction
@@ -186,13 +209,14 @@ __device__ __forceinline__ double nt_exp_core(double x) {
   const int k = static_cast<int>(nt_lo(t));
   double r = fma(-kd, NT_EXP_L_HI, x);
   r = fma(-kd, NT_EXP_L_LO, r);
-  const int j = k & 255;
+  const nt_u32 j = static_cast<nt_u32>(k) & 255u;
   const int m = k >> 8;
   double q = fma(r, NT_EXP_C4, NT_EXP_C3);
   q = fma(r, q, NT_EXP_C2);
   const double p = fma(r * r, q, r);
-  const double th = nt_tables.ex.t[2 * j];
-  const double tl = nt_tables.ex.t[2 * j + 1];
+  const NtPair e = nt_pair(nt_tables.ex.t, j);
+  const double th = e.a;
+  const double tl = e.b;
   return ldexp(th + fma(th, p, tl), m);
 }
 
@@ -210,39 +234,47 @@ __device__ __forceinline__ double nt_exp(double x) {
   return bad ? exp(x) : y;
 }
 
-// -2 ln(u) for a positive normal u, by Tang's table-driven method: u = 2^e x
-// with x in [sqrt(1/2), sqrt(2)), F = x rounded to 8 fractional bits of its
-// binade (rounding the high word at bit 12 moves F = 2 - 2^-8 up to the next
-// binade exactly), ln u = e ln2 + ln F + ln(1 + r), r = (x - F) / F,
-// |r| <= 2^-9. x - F is exact and F = 1 near u = 1, so ln u keeps full
-// relative accuracy there. Tables and constants carry the factor -2 (exact).
-// The exponent comes from u's high word alone, so any biased exponent works
-// (the high word may carry into bit 31 for u near the largest double; the
-// arithmetic is unsigned).
-__device__ __forceinline__ double nt_neg2log(double u) {
-  nt_u32 hx = nt_hi(u) + (0x3FF00000u - 0x3FE6A09Eu);
-  // e = (hx >> 20) - 1023 as a double: the biased exponent in the low word of
-  // 2^52 + (hx >> 20), less 2^52 + 1023 (exact), instead of a conversion
-  const double ed = nt_mk(0x43300000u, hx >> 20) - 0x1.00000000003ffp52;
-  hx = (hx & 0x000FFFFFu) + 0x3FE6A09Eu;
-  const double x = nt_mk(hx, nt_lo(u));
-  const nt_u32 fhi = (hx + 0x800u) & 0xFFFFF000u;
-  const nt_u32 idx = (fhi - 0x3FE6A000u) >> 12;
-  const double r = (x - nt_mk(fhi, 0u)) * nt_tables.lg.inv[idx];  // r' = -2 (x - F) / F
+// Words of a double whose low word is k and whose value is 2^52 + k: less
+// 2^52 (or 2^52 plus an offset, exact) it is k as a double, one v_add_f64 with
+// the high word in a register that stays, in place of a conversion.
+__device__ __forceinline__ double nt_from_u32(nt_u32 k, double offset) { return nt_mk(0x43300000u, k) - offset; }
+
+// -2 ln(v 2^-shift) for a positive normal v, by Tang's table-driven method: v
+// = 2^e x with x in about [3/4, 3/2) (the biased high word carries into the
+// exponent at 3/2 - 2^-9), F = x rounded to 8 fractional bits of its binade,
+// i the double nearest 1/F, ln v = e ln2 - ln i + ln(1 + r), r = x i - 1 in
+// one fma, |r| <= 2^-9. i = 1 around x = 1, so the result keeps full relative
+// accuracy there. Tables and constants carry the factor -2 (exact). The
+// threshold carries the rounding bias of F, so the table index, the exponent
+// and x all come from one sum: six integer instructions and two fp64 ones
+// fewer than a subtraction x - F and its division (nine integer, of which the
+// mask and the rounding of F). The exponent comes from v's high word alone, so
+// any biased exponent works (the high word may carry into bit 31 for v near
+// the largest double; the arithmetic is unsigned).
+__device__ __forceinline__ double nt_neg2log_scaled(double v, int shift) {
+  const nt_u32 hx = nt_hi(v) + 0x80800u;
+  const double ed = nt_from_u32(hx >> 20, 0x1p52 + 1023.0 + shift);
+  const double x = nt_mk((hx & 0x000FFFFFu) + 0x3FE7F800u, nt_lo(v));
+  const nt_u32 idx = (hx >> 12) & 0xFFu;
+  const double r = fma(x, nt_tables.lg.inv[idx], 2.0);  // r' = -2 (x i - 1)
   double q = fma(r, NT_LOGQ_4, NT_LOGQ_3);
   q = fma(r, q, NT_LOGQ_2);
   q = fma(r, q, NT_LOGQ_1);
   q = fma(r, q, NT_LOGQ_0);
-  const double p = fma(r * r, q, r);  // -2 ln(1 + (x - F) / F)
+  const double p = fma(r * r, q, r);  // -2 ln(x i)
   const double hi = fma(ed, NT_M2LN2_HI, nt_tables.lg.hi[idx]);  // exact by the table's layout
   const double lo = fma(ed, NT_M2LN2_LO, nt_tables.lg.lo[idx]) + p;
   return hi + lo;
 }
 
+// -2 ln(u) for a positive normal u.
+__device__ __forceinline__ double nt_neg2log(double u) { return nt_neg2log_scaled(u, 0); }
+
+// c + 1/2 for a 32-bit c, exact: 2^32 times Box-Muller's uniform u = (c + 0.5) * 2^-32.
+__device__ __forceinline__ double nt_u32_half(nt_u32 c) { return nt_from_u32(c, 0x1p52 - 0.5); }
+
 // Box-Muller's -2 ln(u) for u = (c + 0.5) * 2^-32.
-__device__ __forceinline__ double nt_neg2log_u32(nt_u32 c) {
-  return nt_neg2log(fma(static_cast<double>(c), 0x1p-32, 0x1p-33));
-}
+__device__ __forceinline__ double nt_neg2log_u32(nt_u32 c) { return nt_neg2log_scaled(nt_u32_half(c), 32); }
 
 // ln(a) of a LOG node: -1/2 times nt_neg2log (an exact scaling). An argument
 // that is not a positive normal number (zero, subnormal, negative, infinite,
@@ -252,17 +284,16 @@ __device__ __forceinline__ double nt_log_fast(double a, bool& bad) {
   return -0.5 * nt_neg2log(a);
 }
 
-// sqrt(a) for a positive normal finite a: reciprocal square root seed and one
-// coupled Newton step on (sqrt, 1/(2 sqrt)), then a residual correction.
+// sqrt(a) for a positive normal finite a: with the reciprocal square root seed
+// y, g = a y, the residual d = a - g^2 (exact) and e = 1 - g y, sqrt(a) = g + d
+// y (1/2 + 3 e/8) to third order in e (e^3 below 2^-60): half an ulp and
+// little more, one fp64 instruction fewer than a coupled Newton step and a
+// residual correction.
 __device__ __forceinline__ double nt_sqrt_pos(double a) {
   const double y = nt_rsq(a);
-  double g = a * y;
-  double h = 0.5 * y;
-  const double r = fma(-g, h, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
+  const double g = a * y;
   const double d = fma(-g, g, a);
-  return fma(d, h, g);
+  return fma(d * y, fma(fma(-g, y, 1.0), 0.375, 0.5), g);
 }
 
 // 1/b for a DIV node whose numerator is the constant 1, in fp64 tangent
@@ -282,64 +313,53 @@ __device__ __forceinline__ double nt_recip(double b, bool& bad) {
 
 // sin and cos of theta = fl(6.283185307179586 * u) for u = (c + 0.5) * 2^-32.
 // The reference rounds its angle once, and so does this (theta is that
-// rounded product): the per-path results of the Heston tape move by a few
-// 1e-12 when the normals lose that rounding (4.7e-15 at most). The circle is
-// cut in 512 sectors: c = j 2^23 + d with d the sign-extended low 23 bits, so
-// u = j/512 + f exactly, f = (d + 0.5) 2^-32, |f| <= 2^-10 turns. With
-// (S, C) = (sin, cos)(2 pi j/512) from the table, sin(2 pi u) = S cos(2 pi f)
-// + C sin(2 pi f) and cos(2 pi u) = C cos(2 pi f) - S sin(2 pi f), the
-// small-angle parts being polynomials in f. The rounding of theta, eps =
-// theta - 2 pi u, is known exactly (two FMAs) and enters as sin(2 pi f + eps)
-// = sin(2 pi f) + eps to first order (the second-order terms are below
-// 1e-17).
-struct __attribute__((aligned(16))) NtPair {
-  double a, b;
-};
+// rounded product; the scaling by 2^-32 is exact): the per-path results of
+// the Heston tape move by a few 1e-12 when the normals lose that rounding
+// (4.7e-15 at most). The circle is cut in 512 sectors, the sector the top 9
+// bits of c; its table angle a, near the sector's middle, is a multiple of
+// 2^-40, so w = theta - a is exact (for theta below 2^-12, to 2^-60), |w| <=
+// pi/512 + 2^-28, and with (S, C) = (sin, cos)(a), doubles to a few hundredths
+// of an ulp by the choice of a, sin theta = S cos w + C sin w, cos theta = C
+// cos w - S sin w, the small-angle parts being polynomials in w. Reducing the
+// rounded angle itself, in radians, drops the four instructions that would
+// carry its rounding error into a reduction of u in turns (15 fp64
+// instructions against 19), and the errors are 0.58 x 2^-53 at most (1.04
+// with table angles at j/512 turns, their sines and cosines rounded).
 __device__ __forceinline__ void nt_sincos_2pi_u32(nt_u32 c, double& s, double& co) {
-  const int d = static_cast<int>(c << 9) >> 9;
-  // c - d = j 2^23, so its shift by 19 is the byte offset 16 j of the
-  // sector's (sin, cos) pair: one 16-byte load, no masking
-  const nt_u32 off = (c - static_cast<nt_u32>(d)) >> 19;
-  const double f = fma(static_cast<double>(d), 0x1p-32, 0x1p-33);
-  const double t = f * f;
-  double ps = fma(t, NT_SC_S5, NT_SC_S3);
-  ps = fma(t, ps, NT_SC_S1);
-  const double cq = fma(t, NT_SC_C4, NT_SC_C2);
-  const double cm = t * cq;  // cos(2 pi f) - 1
-  const double u = fma(static_cast<double>(c), 0x1p-32, 0x1p-33);
-  const double theta = NT_TWO_PI_D * u;
-  const double eps = fma(NT_TWO_PI_D_ERR, u, -fma(NT_TWO_PI_D, u, -theta));
-  const double sn = fma(f, ps, eps);  // sin(2 pi f) + eps
-  const NtPair sc = *reinterpret_cast<const NtPair*>(reinterpret_cast<const char*>(nt_tables.sc.t) + off);
-  const double S = sc.a;
-  const double C = sc.b;
+#if defined(__clang__)
+#pragma clang fp contract(off)  // theta must be rounded before a is taken off
+#endif
+  const nt_u32 j = c >> 23;
+  const double w = NT_TWO_PI_U32 * nt_u32_half(c) - nt_tables.sc.ang[j];
+  const double t = w * w;
+  const double sn = fma(w * t, fma(t, NT_SC_S5, NT_SC_S3), w);
+  const double cm = t * fma(t, NT_SC_C4, -0.5);  // cos(w) - 1
+  const double S = nt_tables.sc.sin[j];
+  const double C = nt_tables.sc.cos[j];
   s = S + fma(C, sn, S * cm);
   co = C + fma(C, cm, -(S * sn));
 }
 
 // sqrt(a) and the tangent factor 1/(2 sqrt(a)) of a SQRT node, for a = +-0 or
 // a positive normal, where a correctly rounded sqrt and a division take two
-// dozen instructions. nt_sqrt_pos's coupled Newton step and residual
-// correction give the root s; the factor after that step is low by 1.5 e^2
-// (e the seed's relative error, about 2^-24 for v_rsq_f64), the same sign
-// every time, so a Newton step for h = 1/(2 s), h + 2 h (1/2 - s h), brings it
-// to full precision (its error squares): in a carried tangent (a variance
-// process) a one-sided error would compound over the steps. The seed is taken at max(a, 2^-1022), so a = +-0 gives sqrt = a and
-// a large finite factor (the derivative is infinite there; a zero tangent
-// stays zero, as with the capped factor of the libm path). Any other
-// argument (negative, subnormal, infinite, NaN) sets `bad`, and the caller
-// evaluates the path again with device libm.
+// dozen instructions. The root is nt_sqrt_pos's; the factor is y/2 (1 + e/2 +
+// 3 e^2/8) of the same seed and residual, its error that of its roundings, of
+// either sign (in a carried tangent, a variance process, a one-sided error
+// would compound over the steps). The seed is taken at max(a, 2^-1022), so a
+// = +-0 gives sqrt = a and a large finite factor (the derivative is infinite
+// there; a zero tangent stays zero, as with the capped factor of the libm
+// path). Any other argument (negative, subnormal, infinite, NaN) sets `bad`,
+// and the caller evaluates the path again with device libm.
 __device__ __forceinline__ double nt_sqrt_q(double a, double& q, bool& bad) {
   bad |= !nt_zero_or_pos_normal(a);
   const double y = nt_rsq(fmax(a, 0x1p-1022));
-  double g = a * y;
-  double h = 0.5 * y;
-  const double r = fma(-g, h, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  const double s = fma(fma(-g, g, a), h, g);
-  q = fma(h + h, fma(-s, h, 0.5), h);
-  return s;
+  const double g = a * y;
+  const double d = fma(-g, g, a);
+  const double e = fma(-g, y, 1.0);
+  const double p = fma(e, 0.375, 0.5);
+  const double h = 0.5 * y;
+  q = fma(h * e, p, h);
+  return fma(d * y, p, g);
 }
 #else
 __device__ __forceinline__ void nt_tables_load() {}
