@@ -20,6 +20,9 @@
   pi/512 + 2^-28, sin w through w^5 (Taylor, truncation below
   7e-20) and cos w - 1 through w^4 (Taylor, with the w^4 coefficient moved to
   level the error: below 1e-17).
+* the tables and coefficients of the routines that reduce in turns: -2/F and
+  -2 ln F for F = x to 8 fractional bits in [sqrt(1/2), sqrt(2)), (sin, cos)(2
+  pi j / 512), sin and cos polynomials in turns.
 * ln 2 as a double-double; the reference's 2 pi literal.
 All values are computed here with mpmath at 60 digits and rounded once.
 Run: python nablatensor_amd/csrc/gen_math_tables.py
@@ -141,13 +144,40 @@ def main() -> None:
            [("sin", sn, "sin a_j"), ("cos", cs, "cos a_j"), ("ang", ang, "a_j, near 2 pi (j + 1/2) / 512")])
     struct("NtLogTable", "NT_LOG_TABLE_INIT",
            [("inv", inv, "-2 i, i = 1/F rounded"), ("hi", lo_hi, "2 ln i, head"), ("lo", lo_lo, "tail")])
+    # the tables of the routines that reduce in turns (NT_TURN_DRAWS)
+    inv, lo_hi, lo_lo = [], [], []
+    for idx in range(257):
+        F = from_hi(0x3FE6A000 + (idx << 12))
+        inv.append(-2.0 * float(mp.mpf(1) / mp.mpf(F)))
+        l = mp.log(mp.mpf(F))
+        h = head(l, -43)
+        lo_hi.append(-2.0 * h)
+        lo_lo.append(-2.0 * float(l - mp.mpf(h)))
+    assert from_hi(0x3FE6A000 + (150 << 12)) == 1.0 and lo_hi[150] == 0.0
+    lines.append(f"#define NT_TWO_PI_D_ERR {hexd(float(mp.mpf(two_pi_d) - tp))}  /* NT_TWO_PI_D - 2 pi */")
+    for k in (1, 3, 5):
+        lines.append(f"#define NT_TURN_S{k} {hexd(float((-1) ** (k // 2) * tp ** k / mp.factorial(k)))}")
+    c6 = -(tp ** 6) / mp.factorial(6)  # the f^4 coefficient levelled as C4 above, on |f| <= 2^-10 turns
+    turn_c = {2: -(tp ** 2) / 2, 4: tp ** 4 / 24 + beta * c6 * mp.mpf(2) ** -20}
+    for k in (2, 4):
+        lines.append(f"#define NT_TURN_C{k} {hexd(float(turn_c[k]))}")
+    sn = [float(mp.sin(tp * j / 512)) for j in range(512)]
+    cs = [float(mp.cos(tp * j / 512)) for j in range(512)]
+    struct("NtTurnTable", "NT_TURN_TABLE_INIT", [("t", pairs(sn, cs), "t[2j], t[2j+1] = sin, cos of 2 pi j / 512")])
+    struct("NtTurnLogTable", "NT_TURN_LOG_TABLE_INIT",
+           [("inv", inv, "-2 / F"), ("hi", lo_hi, "-2 ln F, head"), ("lo", lo_lo, "tail")])
     lines.append("")
     lines.append("// All tables in one LDS block. Columns that share an index are arrays of their own")
     lines.append("// (one address for all of them), one entry longer than they need: at a distance that")
     lines.append("// is a multiple of 512 bytes two reads become one ds_read2st64_b64, which kept the")
     lines.append("// LDS busy 3.6 times as long as the two (SQ_LDS_IDX_ACTIVE of the Asian kernel).")
+    lines.append("#ifdef NT_TURN_DRAWS")
+    lines.append("struct __attribute__((aligned(16))) NtTables {\n  NtTurnTable sc;\n  NtExpTable ex;\n  NtTurnLogTable lg;\n};")
+    lines.append("#define NT_TABLES_INIT { NT_TURN_TABLE_INIT, NT_EXP_TABLE_INIT, NT_TURN_LOG_TABLE_INIT }")
+    lines.append("#else")
     lines.append("struct __attribute__((aligned(16))) NtTables {\n  NtSinCosTable sc;\n  NtExpTable ex;\n  NtLogTable lg;\n};")
     lines.append("#define NT_TABLES_INIT { NT_SINCOS_TABLE_INIT, NT_EXP_TABLE_INIT, NT_LOG_TABLE_INIT }")
+    lines.append("#endif")
     out = Path(__file__).resolve().parent / "nt_math_tables.h"
     out.write_text("\n".join(lines) + "\n")
     print("wrote", out)

@@ -1491,6 +1491,17 @@ class Emitter {
     }
     return false;
   }
+  // The tape takes the square root of an active value that depends on a draw
+  // (a variance process): see NT_TURN_DRAWS in the skeleton.
+  bool active_sqrt() const {
+    std::vector<char> drawn(t_.n, 0);
+    for (int i = 0; i < t_.n; ++i) {
+      const int ar = is_draw(t_.op[i]) ? 0 : arity(t_.op[i]);
+      drawn[i] = is_draw(t_.op[i]) || (ar >= 1 && drawn[t_.a[i]]) || (ar >= 2 && drawn[t_.b[i]]);
+      if (t_.op[i] == NT_OP_SQRT && t_.active[i] && drawn[i]) return true;
+    }
+    return false;
+  }
   // fp64 tangent kernels with the skeleton's own math take a SQRT node's value
   // and tangent factor from one nt_sqrt_q (a path whose argument it does not
   // cover is evaluated again with device libm).
@@ -3172,6 +3183,7 @@ void Emitter::preamble() {
   o_ << "#pragma clang fp contract(" << (p_.contract ? "fast" : "off") << ")\n";
   if (p_.libm == 1) o_ << "#define NT_DEVICE_LIBM 1\n";
   if (p_.libm == 2) o_ << "#define NT_LIBM_SINCOS 1\n";
+  if (!f32_ && p_.libm != 1 && active_sqrt()) o_ << "#define NT_TURN_DRAWS 1\n";
   o_ << "#include \"nt_skeleton.h\"\n";
   o_ << "typedef " << (f32_ ? "float" : "double") << " real;\n";
   if (fallback()) o_ << "#define NT_HAS_SLOW 1\n";
@@ -3207,6 +3219,7 @@ void Emitter::kernel_head(bool slow) {
   o_ << "  const nt_u64 nt_words = T >> 6;  // lane bitmap words per market\n";
   o_ << "  nt_u64* __restrict__ nt_bits = flags + 1;\n";
   o_ << "  (void)scratch; (void)out_v; (void)out_g; (void)nt_bits; (void)nt_words;\n";
+  if (!slow) o_ << "#ifdef NT_ROWS\n  const nt_u64 nt_t0 = nt_clock();\n#endif\n";
   const int nacc = p_.n_channels * M;
   o_ << "  double acc[" << nacc << "];\n";
   o_ << "  for (int c = 0; c < " << nacc << "; ++c) acc[c] = 0.0;\n";
@@ -3671,7 +3684,14 @@ void Emitter::kernel(bool slow) {
   }
   const int nacc = p_.n_channels * M;
   o_ << "  __shared__ double nt_lds[" << nacc << " * (" << p_.block << " / 64)];\n";
+  if (!slow) {
+    // a small dispatch's blocks write their sums for the host to add
+    std::string bad = "false";
+    for (int m = 0; m < M && fb; ++m) bad = (m ? bad + " || " : std::string()) + "nt_lane_bad" + std::to_string(m);
+    o_ << "#ifdef NT_ROWS\n  nt_block_out<" << nacc << ">(acc, partials, nt_lds, out_v, " << bad << ", nt_t0);\n#else\n";
+  }
   o_ << "  nt_block_store<" << nacc << ">(acc, partials, nt_lds);\n";
+  if (!slow) o_ << "#endif\n";
   o_ << "}\n";
   slow_ = false;
   mlo_ = 0;

@@ -59,8 +59,14 @@ struct nt_exec {
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   double* d_inputs = nullptr;
   double* d_partials = nullptr;
+  char* h_base = nullptr;    // one pinned allocation: the rows, inputs, first sums and flag word below
   double* h_sums = nullptr;  // pinned host rows the finishing kernels write the sums to
+  double* h_grown = nullptr;       // their own allocation once several input sets outgrow the first
   uint32_t* h_deferred = nullptr;  // pinned host word: the finishing pass found flagged lanes (nt_exec_replay)
+  double* h_inputs = nullptr;      // inputs of a small dispatch, read by its kernel from here
+  uint64_t* h_rows = nullptr;      // the blocks' sums of a small dispatch (nt_block_rows)
+  std::vector<double> lane_sums;   // scratch of the host's finishing pass
+  double clock_khz = 0;            // rate of the device clock in the rows
   size_t h_cap = 0;          // doubles in h_sums
   void* d_scratch = nullptr;
   size_t scratch_bytes = 0;  // bytes of d_scratch: the reverse sweep's per-lane tape at the resident grid
@@ -73,7 +79,8 @@ struct nt_exec {
   int cus = 0;          // compute units of the device
   bool fixed_grid = false;  // the caller capped the grid (nt_options.max_blocks)
   std::vector<double> inputs;
-  bool dirty = true;
+  bool dirty = true;        // the inputs are not in d_inputs yet
+  bool from_host = false;   // a small dispatch has read these inputs from h_inputs
   std::map<int, ntr::MarketVariant> markets;  // by set count
   int market_chunk = 0;                       // input sets per multi-market dispatch, 0 until chosen
   double* d_set_inputs = nullptr;             // one input set at a time (reverse-sweep executables)
@@ -106,6 +113,12 @@ size_t flags_bytes_for(uint64_t lanes, int markets);
 // its flag region there (nt_noalloc.hip). Called when an executable is
 // created, so that entry point itself never has to.
 int noalloc_prepare(int dev);
+
+// Whether the executable's sums fit a small dispatch's rows; the wait for the
+// rows of `grid` blocks; and their sums (see nt_rocm.cpp).
+bool rows_fit(const nt_exec* x);
+int await_rows(nt_exec* x, int grid);
+bool finish_rows(nt_exec* x, int grid, double* sums, double& ms);
 
 // Length of each channel's column of partials in a dispatch over `grid`
 // blocks (the skeleton's nt_partial_column): the replay kernel's region of

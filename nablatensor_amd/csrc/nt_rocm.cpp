@@ -58,6 +58,10 @@ using ntr::MarketVariant;
 namespace {
 
 const char* kArch = "gfx950";
+constexpr int kRowBlocks = 512;    // most blocks whose sums the host adds (finish_rows)
+constexpr int kWatchBlocks = 128;  // most blocks whose rows the host watches for, and for how long (await_rows)
+constexpr int kWatchMicros = 1000;
+constexpr uint64_t kUnwritten = 0x7ff5a3c96e1d2b47ull;  // a signalling NaN that no arithmetic gives
 
 // ---- code-object cache ---------------------------------------------------------
 
@@ -377,8 +381,8 @@ nt_exec::~nt_exec() {
   if (stream) (void)hipStreamDestroy(stream);
   if (d_scratch) (void)hipFree(d_scratch);
   if (d_flags) (void)hipFree(d_flags);
-  if (h_sums) (void)hipHostFree(h_sums);
-  if (h_deferred) (void)hipHostFree(h_deferred);
+  if (h_grown) (void)hipHostFree(h_grown);
+  if (h_base) (void)hipHostFree(h_base);
   if (d_partials) (void)hipFree(d_partials);
   if (d_inputs) (void)hipFree(d_inputs);
   for (auto& kv : markets) {
@@ -468,6 +472,68 @@ size_t tape_bytes_per_lane(const nt_exec* x) {
 
 size_t flags_bytes_for(uint64_t lanes, int markets) {
   return (1 + static_cast<size_t>((lanes + 63) / 64) * static_cast<size_t>(std::max(1, markets))) * sizeof(uint64_t);
+}
+
+// A dispatch on at most kRowBlocks blocks writes its blocks' sums to pinned
+// host memory and the host adds them: one launch and one wait, where the
+// finishing pass costs a second launch, its wait for the replay kernel, its
+// own 6 us and the three events that time the two. Measured per dispatch,
+// European call: 1 block 21.2 -> 11 us, 40 blocks 22.7 -> 13.0, 391 blocks
+// 23.6 -> 18.2; 768 blocks 27.2 -> 30.8, where the host's reading of the rows
+// and the blocks' writes over PCIe cost more than the pass.
+bool rows_fit(const nt_exec* x) { return x->low.plan.n_channels <= 128; }
+
+// Waits for the rows of a dispatch on at most kWatchBlocks blocks. Every word
+// was set to kUnwritten before the launch; the first kWatchMicros the host
+// watches for the words themselves, which arrive before the runtime sees the
+// kernel's end. Measured per dispatch, draining the stream against watching:
+// 40 blocks 16.3 and 13.0 us, 79 blocks 24.2 and 22.2, 391 blocks 18.2 and
+// 20.1 (the European call and the 64-fixing Asian). After that (a long kernel,
+// a failed one, a sum that is that very NaN) the stream is drained as usual.
+int await_rows(nt_exec* x, int grid) {
+  const size_t words = static_cast<size_t>(grid) * (static_cast<size_t>(x->low.plan.n_channels) + 2);
+  const auto t0 = std::chrono::steady_clock::now();
+  size_t w = grid <= kWatchBlocks ? 0 : words + 1;
+  for (unsigned spins = 1; w <= words; ++spins) {
+    while (w < words && __atomic_load_n(x->h_rows + w, __ATOMIC_ACQUIRE) != kUnwritten) ++w;
+    if (w == words) return NT_OK;
+    if ((spins & 63) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(kWatchMicros)) break;
+    __builtin_ia32_pause();
+  }
+  NT_HIP(hipStreamSynchronize(x->stream), "hipStreamSynchronize");
+  return NT_OK;
+}
+
+// The sums of a small dispatch from its blocks' rows, in nt_finish's order:
+// lane l of 64 adds the blocks 8 (l + 64 k) + x, x = 0..7 the outer loop and k
+// the inner (kRowBlocks is within one batch of the pass), and the lanes are
+// added by the wave's butterfly. Returns whether a block had a lane with paths
+// for the exception kernel; `ms` is the time from the first block's start to
+// the last block's end on the device clock.
+bool finish_rows(nt_exec* x, int grid, double* sums, double& ms) {
+  const int nch = x->low.plan.n_channels, stride = nch + 2;
+  double* lane = x->lane_sums.data();  // [64][nch]
+  std::fill_n(lane, static_cast<size_t>(64) * nch, 0.0);
+  uint64_t first = ~0ull, last = 0, bad = 0;
+  for (int cls = 0; cls < 8; ++cls) {
+    for (int b = cls; b < grid; b += 8) {  // k = b / 512 ascends within a lane
+      const uint64_t* row = x->h_rows + static_cast<size_t>(b) * stride;
+      first = std::min(first, row[0]);
+      last = std::max(last, row[1] >> 1);
+      bad |= row[1] & 1;
+      const double* v = reinterpret_cast<const double*>(row + 2);
+      double* to = lane + static_cast<size_t>((b >> 3) & 63) * nch;
+      for (int c = 0; c < nch; ++c) to[c] += v[c];
+    }
+  }
+  for (int m = 32; m >= 1; m >>= 1) {
+    for (int l = 0; l < m; ++l) {
+      for (int c = 0; c < nch; ++c) lane[static_cast<size_t>(l) * nch + c] += lane[static_cast<size_t>(l + m) * nch + c];
+    }
+  }
+  std::copy_n(lane, nch, sums);
+  ms = static_cast<double>(std::max<uint64_t>(last > first ? last - first : 0, 1)) / x->clock_khz;
+  return bad != 0;
 }
 
 int partial_rows(int grid) { return 16 * ((grid + 7) / 8); }
@@ -616,11 +682,23 @@ int nt_exec_create(const nt_tape* tape, const nt_options* options, nt_exec** out
   NT_HIP(hipMalloc(&x->d_partials,
                    sizeof(double) * static_cast<size_t>(ntr::partial_rows(x->grid_cap)) * nch),
          "hipMalloc(partials)");
-  NT_HIP(hipHostMalloc(reinterpret_cast<void**>(&x->h_sums), sizeof(double) * nch, hipHostMallocDefault),
-         "hipHostMalloc(sums)");
-  NT_HIP(hipHostMalloc(reinterpret_cast<void**>(&x->h_deferred), sizeof(uint32_t), hipHostMallocDefault),
-         "hipHostMalloc(deferred)");
+  const size_t row_words = ntr::rows_fit(x.get()) ? static_cast<size_t>(kRowBlocks) * (nch + 2) : 0;
+  const size_t in_words = static_cast<size_t>(std::max(1, x->low.ir.n_in));
+  NT_HIP(hipHostMalloc(reinterpret_cast<void**>(&x->h_base), sizeof(uint64_t) * (row_words + in_words + nch + 1),
+                       hipHostMallocDefault),
+         "hipHostMalloc(rows, inputs, sums)");
+  x->h_rows = row_words ? reinterpret_cast<uint64_t*>(x->h_base) : nullptr;
+  x->h_inputs = reinterpret_cast<double*>(x->h_base) + row_words;
+  x->h_sums = x->h_inputs + in_words;
+  x->h_deferred = reinterpret_cast<uint32_t*>(x->h_sums + nch);
   x->h_cap = static_cast<size_t>(nch);
+  x->lane_sums.assign(row_words ? static_cast<size_t>(64) * nch : 0, 0.0);
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, x->dev) != hipSuccess || khz <= 0) {
+    (void)hipGetLastError();
+    khz = 100000;
+  }
+  x->clock_khz = khz;
   const size_t scratch = ntr::tape_bytes_per_lane(x.get()) * x->grid_cap * x->low.plan.block;
   if (scratch > 0) NT_HIP(hipMalloc(&x->d_scratch, scratch), "hipMalloc(scratch)");
   x->scratch_bytes = scratch;
@@ -642,6 +720,7 @@ int nt_exec_set_inputs(nt_exec* x, const double* inputs, int32_t n) {
   if (n != x->low.ir.n_in || (n > 0 && !inputs)) return fail(NT_E_INVALID, "expected one value per tape input");
   x->inputs.assign(inputs, inputs + n);
   x->dirty = true;
+  x->from_host = false;
   return NT_OK;
 }
 
@@ -679,16 +758,20 @@ static int launch_kernel(nt_exec* x, hipFunction_t fn, hipFunction_t fn_slow, do
                                offset, seed, out_v, out_g, grid, between);
 }
 
+static int upload_inputs(nt_exec* x) {
+  if (x->dirty && !x->inputs.empty()) {
+    NT_HIP(hipMemcpyAsync(x->d_inputs, x->inputs.data(), sizeof(double) * x->inputs.size(), hipMemcpyHostToDevice,
+                          x->stream),
+           "hipMemcpyAsync(inputs)");
+  }
+  x->dirty = false;
+  return NT_OK;
+}
+
 static int launch_replay(nt_exec* x, hipFunction_t fn, hipFunction_t fn_slow, uint64_t paths, uint64_t offset,
                          uint64_t seed, double* out_v, double* out_g, int& grid, hipEvent_t between = nullptr) {
-  if (x->dirty) {
-    if (!x->inputs.empty()) {
-      NT_HIP(hipMemcpyAsync(x->d_inputs, x->inputs.data(), sizeof(double) * x->inputs.size(), hipMemcpyHostToDevice,
-                            x->stream),
-             "hipMemcpyAsync(inputs)");
-    }
-    x->dirty = false;
-  }
+  const int rc = upload_inputs(x);
+  if (rc != NT_OK) return rc;
   return launch_kernel(x, fn, fn_slow, x->d_inputs, x->d_partials, x->low.plan.n_channels, 1, paths, offset, seed,
                        out_v, out_g, grid, between);
 }
@@ -701,6 +784,56 @@ static int launch_finish(nt_exec* x, hipFunction_t fn, hipFunction_t fn_slow, do
                                fn_slow ? x->d_flags : nullptr);
 }
 
+// A dispatch on at most kRowBlocks blocks: one launch, the blocks' sums added
+// by the host. Inputs bound since the last dispatch are read by the kernel
+// from pinned memory, with no copy; a second such dispatch on the same inputs
+// uploads them, and later ones read device memory.
+static int replay_rows(nt_exec* x, int grid, uint64_t paths, uint64_t offset, uint64_t seed, double* sums,
+                       double* timing, std::chrono::steady_clock::time_point t0) {
+  const int nch = x->low.plan.n_channels;
+  const double* d_in = x->d_inputs;
+  if (x->dirty && !x->inputs.empty()) {
+    if (!x->from_host) {
+      std::copy(x->inputs.begin(), x->inputs.end(), x->h_inputs);
+      x->from_host = true;
+      d_in = x->h_inputs;
+    } else {
+      const int rc = upload_inputs(x);
+      if (rc != NT_OK) return rc;
+    }
+  }
+  const bool watch = grid <= kWatchBlocks;
+  if (watch) std::fill_n(x->h_rows, static_cast<size_t>(grid) * (nch + 2), kUnwritten);
+  int rc = ntr::launch_kernel_on(x, x->stream, x->fn, nullptr, d_in, x->d_partials, nch, x->d_scratch, x->d_flags,
+                                 paths, offset, seed,
+                                 reinterpret_cast<double*>(reinterpret_cast<uintptr_t>(x->h_rows) | (watch ? 1 : 0)),
+                                 nullptr, grid);
+  if (rc == NT_OK) rc = ntr::await_rows(x, grid);
+  if (rc != NT_OK) return rc;
+  double replay_ms = 0;
+  float rest_ms = 0;
+  if (ntr::finish_rows(x, grid, sums, replay_ms) && x->fn_slow) {
+    // Some lane left its paths to the exception kernel: it and the finishing
+    // pass follow, on the partials that the blocks wrote beside their rows.
+    NT_HIP(hipEventRecord(x->ev[0], x->stream), "hipEventRecord");
+    rc = ntr::launch_slow_on(x, x->stream, x->fn_slow, d_in, x->d_partials, nch, x->d_scratch, x->d_flags, paths,
+                             offset, seed, nullptr, nullptr, grid);
+    if (rc != NT_OK) return rc;
+    rc = launch_finish(x, x->fn_finish, x->fn_slow, x->d_partials, grid, nch, x->h_sums);
+    if (rc != NT_OK) return rc;
+    NT_HIP(hipEventRecord(x->ev[2], x->stream), "hipEventRecord");
+    NT_HIP(hipStreamSynchronize(x->stream), "hipStreamSynchronize");
+    NT_HIP(hipEventElapsedTime(&rest_ms, x->ev[0], x->ev[2]), "hipEventElapsedTime");
+    std::memcpy(sums, x->h_sums, sizeof(double) * nch);
+  }
+  if (timing) {
+    timing[0] = replay_ms + rest_ms;
+    timing[1] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    timing[2] = replay_ms;
+  }
+  return NT_OK;
+}
+
 int nt_exec_replay(nt_exec* x, uint64_t paths, uint64_t offset, uint64_t seed, double* sums, int32_t n_sums,
                    double* timing) {
   if (!x) return fail(NT_E_CLOSED, "executable is closed");
@@ -709,6 +842,10 @@ int nt_exec_replay(nt_exec* x, uint64_t paths, uint64_t offset, uint64_t seed, d
   if (!sums || n_sums != nch) return fail(NT_E_INVALID, "sums must hold n_outputs * (2 + n_inputs) doubles");
   const auto t0 = std::chrono::steady_clock::now();
   NT_HIP(hipSetDevice(x->dev), "hipSetDevice");
+  if (x->h_rows) {
+    const int blocks = grid_for(x, paths);
+    if (blocks <= kRowBlocks) return replay_rows(x, blocks, paths, offset, seed, sums, timing, t0);
+  }
   NT_HIP(hipEventRecord(x->ev[0], x->stream), "hipEventRecord");
   int grid = 0;
   // The exception kernel runs only when the replay kernel left paths to it:
@@ -848,8 +985,8 @@ int nt_exec_replay_many(nt_exec* x, const double* input_sets, int32_t markets, u
     double* grown = nullptr;
     NT_HIP(hipHostMalloc(reinterpret_cast<void**>(&grown), sizeof(double) * need, hipHostMallocDefault),
            "hipHostMalloc(sums)");
-    (void)hipHostFree(x->h_sums);
-    x->h_sums = grown;
+    if (x->h_grown) (void)hipHostFree(x->h_grown);
+    x->h_sums = x->h_grown = grown;
     x->h_cap = need;
   }
   NT_HIP(hipEventRecord(x->ev[0], x->stream), "hipEventRecord");

@@ -234,6 +234,93 @@ __device__ __forceinline__ double nt_exp(double x) {
   return bad ? exp(x) : y;
 }
 
+#ifdef NT_TURN_DRAWS
+// The routines of tapes whose step takes the square root of an active value (a
+// variance): near its floor such a value multiplies the last bit of a draw by
+// 1 / (2 sqrt v), and one path of 10^7 can move a derivative's sum by 3e-11 of
+// itself. These tapes keep the rounding of their draws and roots, from the
+// routines below; every other tape takes the shorter ones after them.
+
+// -2 ln(u) for a positive normal u, by Tang's method with F = x rounded to 8
+// fractional bits of its binade and r = (x - F) / F, x - F exact.
+__device__ __forceinline__ double nt_neg2log(double u) {
+  nt_u32 hx = nt_hi(u) + (0x3FF00000u - 0x3FE6A09Eu);
+  // e = (hx >> 20) - 1023 as a double: the biased exponent in the low word of
+  // 2^52 + (hx >> 20), less 2^52 + 1023 (exact), instead of a conversion
+  const double ed = nt_mk(0x43300000u, hx >> 20) - 0x1.00000000003ffp52;
+  hx = (hx & 0x000FFFFFu) + 0x3FE6A09Eu;
+  const double x = nt_mk(hx, nt_lo(u));
+  const nt_u32 fhi = (hx + 0x800u) & 0xFFFFF000u;
+  const nt_u32 idx = (fhi - 0x3FE6A000u) >> 12;
+  const double r = (x - nt_mk(fhi, 0u)) * nt_tables.lg.inv[idx];  // r' = -2 (x - F) / F
+  double q = fma(r, NT_LOGQ_4, NT_LOGQ_3);
+  q = fma(r, q, NT_LOGQ_2);
+  q = fma(r, q, NT_LOGQ_1);
+  q = fma(r, q, NT_LOGQ_0);
+  const double p = fma(r * r, q, r);  // -2 ln(1 + (x - F) / F)
+  const double hi = fma(ed, NT_M2LN2_HI, nt_tables.lg.hi[idx]);  // exact by the table's layout
+  const double lo = fma(ed, NT_M2LN2_LO, nt_tables.lg.lo[idx]) + p;
+  return hi + lo;
+}
+
+
+__device__ __forceinline__ double nt_neg2log_u32(nt_u32 c) {
+  return nt_neg2log(fma(static_cast<double>(c), 0x1p-32, 0x1p-33));
+}
+
+// sqrt(a) for a positive normal finite a: one coupled Newton step on (sqrt,
+// 1/(2 sqrt)), then a residual correction.
+__device__ __forceinline__ double nt_sqrt_pos(double a) {
+  const double y = nt_rsq(a);
+  double g = a * y;
+  double h = 0.5 * y;
+  const double r = fma(-g, h, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  const double d = fma(-g, g, a);
+  return fma(d, h, g);
+}
+
+// sin and cos of theta = fl(6.283185307179586 * u), reduced in turns: c = j 2^23
+// + d, u = j/512 + f exactly, the rounding of theta (two FMAs) added to
+// sin(2 pi f).
+__device__ __forceinline__ void nt_sincos_2pi_u32(nt_u32 c, double& s, double& co) {
+  const int d = static_cast<int>(c << 9) >> 9;
+  // c - d = j 2^23, so its shift by 19 is the byte offset 16 j of the
+  // sector's (sin, cos) pair: one 16-byte load, no masking
+  const nt_u32 off = (c - static_cast<nt_u32>(d)) >> 19;
+  const double f = fma(static_cast<double>(d), 0x1p-32, 0x1p-33);
+  const double t = f * f;
+  double ps = fma(t, NT_TURN_S5, NT_TURN_S3);
+  ps = fma(t, ps, NT_TURN_S1);
+  const double cq = fma(t, NT_TURN_C4, NT_TURN_C2);
+  const double cm = t * cq;  // cos(2 pi f) - 1
+  const double u = fma(static_cast<double>(c), 0x1p-32, 0x1p-33);
+  const double theta = NT_TWO_PI_D * u;
+  const double eps = fma(NT_TWO_PI_D_ERR, u, -fma(NT_TWO_PI_D, u, -theta));
+  const double sn = fma(f, ps, eps);  // sin(2 pi f) + eps
+  const NtPair sc = *reinterpret_cast<const NtPair*>(reinterpret_cast<const char*>(nt_tables.sc.t) + off);
+  const double S = sc.a;
+  const double C = sc.b;
+  s = S + fma(C, sn, S * cm);
+  co = C + fma(C, cm, -(S * sn));
+}
+
+// sqrt(a) and 1/(2 sqrt(a)): the coupled step, the residual correction and a
+// Newton step on the factor; arguments and `bad` as in the routine below.
+__device__ __forceinline__ double nt_sqrt_q(double a, double& q, bool& bad) {
+  bad |= !nt_zero_or_pos_normal(a);
+  const double y = nt_rsq(fmax(a, 0x1p-1022));
+  double g = a * y;
+  double h = 0.5 * y;
+  const double r = fma(-g, h, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  const double s = fma(fma(-g, g, a), h, g);
+  q = fma(h + h, fma(-s, h, 0.5), h);
+  return s;
+}
+#else
 // Words of a double whose low word is k and whose value is 2^52 + k: less
 // 2^52 (or 2^52 plus an offset, exact) it is k as a double, one v_add_f64 with
 // the high word in a register that stays, in place of a conversion.
@@ -276,14 +363,6 @@ __device__ __forceinline__ double nt_u32_half(nt_u32 c) { return nt_from_u32(c, 
 // Box-Muller's -2 ln(u) for u = (c + 0.5) * 2^-32.
 __device__ __forceinline__ double nt_neg2log_u32(nt_u32 c) { return nt_neg2log_scaled(nt_u32_half(c), 32); }
 
-// ln(a) of a LOG node: -1/2 times nt_neg2log (an exact scaling). An argument
-// that is not a positive normal number (zero, subnormal, negative, infinite,
-// NaN) sets `bad`, and the path is evaluated again with device libm.
-__device__ __forceinline__ double nt_log_fast(double a, bool& bad) {
-  bad |= !nt_pos_normal(a);
-  return -0.5 * nt_neg2log(a);
-}
-
 // sqrt(a) for a positive normal finite a: with the reciprocal square root seed
 // y, g = a y, the residual d = a - g^2 (exact) and e = 1 - g y, sqrt(a) = g + d
 // y (1/2 + 3 e/8) to third order in e (e^3 below 2^-60): half an ulp and
@@ -294,21 +373,6 @@ __device__ __forceinline__ double nt_sqrt_pos(double a) {
   const double g = a * y;
   const double d = fma(-g, g, a);
   return fma(d * y, fma(fma(-g, y, 1.0), 0.375, 0.5), g);
-}
-
-// 1/b for a DIV node whose numerator is the constant 1, in fp64 tangent
-// kernels (the value is also the node's tangent factor): the v_rcp_f64 seed
-// and two Newton steps give it within an ulp, where a correctly rounded
-// division takes eleven instructions. For |b| outside [2^-1022, 2^1022]
-// (zero, subnormal, huge, infinite, NaN) `bad` is set and the caller
-// evaluates the path again with device libm.
-__device__ __forceinline__ double nt_recip(double b, bool& bad) {
-  bad |= !(fabs(b) >= 0x1p-1022 && fabs(b) <= 0x1p1022);
-  double y = nt_rcp(b);
-  double e = fma(-b, y, 1.0);
-  y = fma(y, e, y);
-  e = fma(-b, y, 1.0);
-  return fma(y, e, y);
 }
 
 // sin and cos of theta = fl(6.283185307179586 * u) for u = (c + 0.5) * 2^-32.
@@ -361,6 +425,31 @@ __device__ __forceinline__ double nt_sqrt_q(double a, double& q, bool& bad) {
   q = fma(h * e, p, h);
   return fma(d * y, p, g);
 }
+#endif  // NT_TURN_DRAWS
+
+// ln(a) of a LOG node: -1/2 times nt_neg2log (an exact scaling). An argument
+// that is not a positive normal number (zero, subnormal, negative, infinite,
+// NaN) sets `bad`, and the path is evaluated again with device libm.
+__device__ __forceinline__ double nt_log_fast(double a, bool& bad) {
+  bad |= !nt_pos_normal(a);
+  return -0.5 * nt_neg2log(a);
+}
+
+// 1/b for a DIV node whose numerator is the constant 1, in fp64 tangent
+// kernels (the value is also the node's tangent factor): the v_rcp_f64 seed
+// and two Newton steps give it within an ulp, where a correctly rounded
+// division takes eleven instructions. For |b| outside [2^-1022, 2^1022]
+// (zero, subnormal, huge, infinite, NaN) `bad` is set and the caller
+// evaluates the path again with device libm.
+__device__ __forceinline__ double nt_recip(double b, bool& bad) {
+  bad |= !(fabs(b) >= 0x1p-1022 && fabs(b) <= 0x1p1022);
+  double y = nt_rcp(b);
+  double e = fma(-b, y, 1.0);
+  y = fma(y, e, y);
+  e = fma(-b, y, 1.0);
+  return fma(y, e, y);
+}
+
 #else
 __device__ __forceinline__ void nt_tables_load() {}
 __device__ __forceinline__ double nt_exp(double x) { return exp(x); }
@@ -515,6 +604,55 @@ __device__ __forceinline__ void nt_block_store(const double (&acc)[NCH], double*
     double s = 0.0;
     for (int w = 0; w < waves; ++w) s += lds[c * waves + w];
     partials[static_cast<nt_u64>(c) * nt_partial_column(gridDim.x) + nt_partial_slot(blockIdx.x, gridDim.x)] = s;
+  }
+}
+
+// nt_block_store for the replay kernel, which may leave its blocks' sums to
+// the host: with `rows` set (pinned host memory, NCH + 2 words a block) row b
+// gets block b's first and last clock, the latter shifted up by one with the
+// lowest bit set when a lane of the block left paths to the exception kernel,
+// then its NCH sums. The host adds them in nt_finish's order, which saves a
+// small dispatch the second launch, the events around it and its wait for the
+// first (the partials are there too, for when the exception kernel has to
+// run). The lowest bit of `rows` says that the host watches for the words one
+// by one while the kernel ends: each is then a store of its own to system
+// scope. Otherwise the host reads them after the kernel's end, and a wave's
+// plain stores leave as whole lines (391 blocks of 9 words: 97 us per weekday
+// Asian dispatch against 102).
+#ifndef NT_DUMP_PATHS
+#define NT_ROWS 1
+#endif
+__device__ __forceinline__ nt_u64 nt_clock() { return __builtin_amdgcn_s_memrealtime(); }
+template <typename T>
+__device__ __forceinline__ void nt_to_host(T* at, T v, bool watched) {
+  if (watched) __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else *at = v;
+}
+template <int NCH>
+__device__ __forceinline__ void nt_block_out(const double (&acc)[NCH], double* __restrict__ partials, double* lds,
+                                             double* __restrict__ rows, bool bad, nt_u64 started) {
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int waves = blockDim.x >> 6;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const double w = nt_wave_sum(acc[c]);
+    if (lane == 0) lds[c * waves + wave] = w;
+  }
+  const nt_u64 any = __syncthreads_or(bad) ? 1 : 0;
+  const bool watched = (reinterpret_cast<nt_u64>(rows) & 1) != 0;
+  double* row = reinterpret_cast<double*>(reinterpret_cast<nt_u64>(rows) & ~1ull) +
+                static_cast<nt_u64>(blockIdx.x) * (NCH + 2);
+  double* slot = partials + nt_partial_slot(blockIdx.x, gridDim.x);
+  for (int c = threadIdx.x; c < NCH; c += blockDim.x) {
+    double s = 0.0;
+    for (int w = 0; w < waves; ++w) s += lds[c * waves + w];
+    slot[c * nt_partial_column(gridDim.x)] = s;
+    if (rows) nt_to_host(row + 2 + c, s, watched);
+  }
+  if (rows && threadIdx.x == 0) {
+    nt_to_host(reinterpret_cast<nt_u64*>(row), started, watched);
+    nt_to_host(reinterpret_cast<nt_u64*>(row) + 1, (nt_clock() << 1) | any, watched);
   }
 }
 
