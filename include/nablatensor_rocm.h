@@ -97,7 +97,9 @@ typedef struct nt_options {
                                fp32, plus the fused exponent of a step's multiplicative carry, whose value is
                                rebuilt from a product of factors anyway, the fp64 tangent loop's sums of products
                                of values with no tangent, such as correlated normals, and a carry's exponent sum
-                               taken as N p + r S after the loop), 1 on, -1 off (every product and sum of a node
+                               taken as N p + r S after the loop, and the body of a reverse-swept fp64 step loop
+                               with libm = 0 on a tape that takes no square root of an active value that depends
+                               on a draw), 1 on, -1 off (every product and sum of a node
                                rounded separately). The skeleton's math routines and the tangent rules use
                                explicit fma either way */
   int32_t libm;             /* fp64 Box-Muller: 0 the skeleton's own log/sqrt/sincos, 1 device libm, 2 own log/sqrt + libm sincos */
