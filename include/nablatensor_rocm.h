@@ -178,7 +178,7 @@ int nt_exec_set_inputs(nt_exec *exec, const double *inputs, int32_t n);
  * when built price-only), the AadTotals fields (AadTotals.java:30-40); n_sums
  * must be n_outputs * (2 + n_inputs). timing (nullable) receives {kernel_ms, wall_ms}: kernel_ms from
  * HIP events around the replay and finishing kernels on the executable's
- * stream (a dispatch on at most 512 blocks has no finishing kernel: the host
+ * stream (a dispatch on few blocks, 512 at most, has no finishing kernel: the host
  * adds the blocks' sums, in the same order, and kernel_ms is the replay
  * kernel's time by the device's clock, from its first block's start to its
  * last block's end), wall_ms from entry to sums on the host. Replaces

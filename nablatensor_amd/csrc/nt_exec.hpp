@@ -114,9 +114,9 @@ size_t flags_bytes_for(uint64_t lanes, int markets);
 // created, so that entry point itself never has to.
 int noalloc_prepare(int dev);
 
-// Whether the executable's sums fit a small dispatch's rows; the wait for the
+// Whether a dispatch of `grid` blocks is a small one; the wait for the
 // rows of `grid` blocks; and their sums (see nt_rocm.cpp).
-bool rows_fit(const nt_exec* x);
+bool rows_fit(const nt_exec* x, int grid);
 int await_rows(nt_exec* x, int grid);
 bool finish_rows(nt_exec* x, int grid, double* sums, double& ms);
 

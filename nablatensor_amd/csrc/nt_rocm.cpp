@@ -59,6 +59,8 @@ namespace {
 
 const char* kArch = "gfx950";
 constexpr int kRowBlocks = 512;    // most blocks whose sums the host adds (finish_rows)
+constexpr size_t kRowWords = 4608;  // most words of their rows (rows_fit)
+constexpr size_t kRowChannels = 128;  // and most sums of one (the host adds 64 lanes of them)
 constexpr int kWatchBlocks = 128;  // most blocks whose rows the host watches for, and for how long (await_rows)
 constexpr int kWatchMicros = 1000;
 constexpr uint64_t kUnwritten = 0x7ff5a3c96e1d2b47ull;  // a signalling NaN that no arithmetic gives
@@ -474,14 +476,19 @@ size_t flags_bytes_for(uint64_t lanes, int markets) {
   return (1 + static_cast<size_t>((lanes + 63) / 64) * static_cast<size_t>(std::max(1, markets))) * sizeof(uint64_t);
 }
 
-// A dispatch on at most kRowBlocks blocks writes its blocks' sums to pinned
-// host memory and the host adds them: one launch and one wait, where the
-// finishing pass costs a second launch, its wait for the replay kernel, its
-// own 6 us and the three events that time the two. Measured per dispatch,
-// European call: 1 block 21.2 -> 11 us, 40 blocks 22.7 -> 13.0, 391 blocks
-// 23.6 -> 18.2; 768 blocks 27.2 -> 30.8, where the host's reading of the rows
-// and the blocks' writes over PCIe cost more than the pass.
-bool rows_fit(const nt_exec* x) { return x->low.plan.n_channels <= 128; }
+// A dispatch on at most kRowBlocks blocks, with at most kRowWords words of
+// rows, writes its blocks' sums to pinned host memory and the host adds them:
+// one launch and one wait, where the finishing pass costs a second launch, its
+// wait for the replay kernel, its own 6 us and the three events that time the
+// two. Measured per dispatch, European call (9 words a block): 1 block 21.2 ->
+// 11 us, 40 blocks 22.7 -> 13.0, 391 blocks 23.6 -> 18.2; 768 blocks (6,912
+// words) 27.2 -> 30.8, where the host's reading of the rows and the blocks'
+// writes over PCIe cost more than the pass, as on a worst-of's 347 blocks of
+// 19 words (6,593): 35.9 -> 37.0 us.
+bool rows_fit(const nt_exec* x, int grid) {
+  const size_t nch = static_cast<size_t>(x->low.plan.n_channels);
+  return nch <= kRowChannels && grid <= kRowBlocks && static_cast<size_t>(grid) * (nch + 2) <= kRowWords;
+}
 
 // Waits for the rows of a dispatch on at most kWatchBlocks blocks. Every word
 // was set to kUnwritten before the launch; the first kWatchMicros the host
@@ -682,17 +689,17 @@ int nt_exec_create(const nt_tape* tape, const nt_options* options, nt_exec** out
   NT_HIP(hipMalloc(&x->d_partials,
                    sizeof(double) * static_cast<size_t>(ntr::partial_rows(x->grid_cap)) * nch),
          "hipMalloc(partials)");
-  const size_t row_words = ntr::rows_fit(x.get()) ? static_cast<size_t>(kRowBlocks) * (nch + 2) : 0;
+  const size_t row_words = std::min(kRowWords, static_cast<size_t>(kRowBlocks) * (nch + 2));
   const size_t in_words = static_cast<size_t>(std::max(1, x->low.ir.n_in));
   NT_HIP(hipHostMalloc(reinterpret_cast<void**>(&x->h_base), sizeof(uint64_t) * (row_words + in_words + nch + 1),
                        hipHostMallocDefault),
          "hipHostMalloc(rows, inputs, sums)");
-  x->h_rows = row_words ? reinterpret_cast<uint64_t*>(x->h_base) : nullptr;
+  x->h_rows = reinterpret_cast<uint64_t*>(x->h_base);
   x->h_inputs = reinterpret_cast<double*>(x->h_base) + row_words;
   x->h_sums = x->h_inputs + in_words;
   x->h_deferred = reinterpret_cast<uint32_t*>(x->h_sums + nch);
   x->h_cap = static_cast<size_t>(nch);
-  x->lane_sums.assign(row_words ? static_cast<size_t>(64) * nch : 0, 0.0);
+  x->lane_sums.assign(static_cast<size_t>(nch) <= kRowChannels ? static_cast<size_t>(64) * nch : 0, 0.0);
   int khz = 0;
   if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, x->dev) != hipSuccess || khz <= 0) {
     (void)hipGetLastError();
@@ -784,7 +791,7 @@ static int launch_finish(nt_exec* x, hipFunction_t fn, hipFunction_t fn_slow, do
                                fn_slow ? x->d_flags : nullptr);
 }
 
-// A dispatch on at most kRowBlocks blocks: one launch, the blocks' sums added
+// A dispatch whose rows fit (rows_fit): one launch, the blocks' sums added
 // by the host. Inputs bound since the last dispatch are read by the kernel
 // from pinned memory, with no copy; a second such dispatch on the same inputs
 // uploads them, and later ones read device memory.
@@ -842,10 +849,8 @@ int nt_exec_replay(nt_exec* x, uint64_t paths, uint64_t offset, uint64_t seed, d
   if (!sums || n_sums != nch) return fail(NT_E_INVALID, "sums must hold n_outputs * (2 + n_inputs) doubles");
   const auto t0 = std::chrono::steady_clock::now();
   NT_HIP(hipSetDevice(x->dev), "hipSetDevice");
-  if (x->h_rows) {
-    const int blocks = grid_for(x, paths);
-    if (blocks <= kRowBlocks) return replay_rows(x, blocks, paths, offset, seed, sums, timing, t0);
-  }
+  const int blocks = grid_for(x, paths);
+  if (ntr::rows_fit(x, blocks)) return replay_rows(x, blocks, paths, offset, seed, sums, timing, t0);
   NT_HIP(hipEventRecord(x->ev[0], x->stream), "hipEventRecord");
   int grid = 0;
   // The exception kernel runs only when the replay kernel left paths to it:
