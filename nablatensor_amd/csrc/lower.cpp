@@ -1172,7 +1172,7 @@ class Emitter {
   // (a volatility polynomial's Horner scheme) at one wave per SIMD, so an fma
   // in place of a multiply and an add shortens the chain as well as the count.
   // The local-volatility Asian (24 coefficients, 2x10^6 paths): 8.49 ms and 386
-  // VGPRs -> 7.16 ms and 338, with first contributions stored (fresh_).
+  // VGPRs -> 7.16 ms and 336, with first contributions stored (fresh_).
   // Tapes that take the square root of an active drawn value keep their
   // rounding (NT_TURN_DRAWS).
   bool rev_fused_ = false;
