@@ -1355,7 +1355,7 @@ class Emitter {
   // reads for something else too)
   std::vector<char> dsum_, hoist_, after_;
   void plan_draw_sums();
-  bool linear_form(int pos, double scale, double& offset, std::vector<char>& draws) const;
+  std::vector<char> linear_forms() const;
   void hoisted_step();
   std::string body_rhs(int u, int j, const std::string& x, const std::string& y) const;
   void draw_sum(int U, int u, int j, std::map<std::pair<int, int>, std::string>& pairs,
@@ -2657,42 +2657,63 @@ void Emitter::plan_geo_affine() {
   }
 }
 
-// Whether scale x (the value of loop position pos) is a linear form of the
-// step's draws: marks them in `draws` and adds its constant term to `offset`.
-bool Emitter::linear_form(int pos, double scale, double& offset, std::vector<char>& draws) const {
-  const int op = t_.op[L_.start + pos];
-  if (!std::isfinite(scale)) return false;
-  if (is_draw(op)) {
-    draws[pos] = 1;
-    return true;
-  }
-  if (t_.active[L_.start + pos]) return false;
+// Per loop position, whether its value is a linear form of the step's draws
+// with literal coefficients and no constant term. One pass in the step's order,
+// so a value that many others read is looked at once.
+std::vector<char> Emitter::linear_forms() const {
+  const int P = L_.period;
+  std::vector<char> linear(P, 0);
+  std::vector<double> size(P, 0.0);  // bounds the coefficients: they stay finite
   auto literal = [&](int kind, int ref, double& v) {
     const int node = kind == ARG_BODY ? L_.start + ref : kind == ARG_INV ? ref : -1;
     if (node < 0 || t_.op[node] != NT_OP_CONST || (kind == ARG_BODY && L_.table_lit(ref))) return false;
     v = t_.c[node];
     return true;
   };
-  auto operand = [&](int kind, int ref, double by) {
-    double v = 0;
-    if (literal(kind, ref, v)) {
-      offset += by * v;
-      return true;
+  for (int j = 0; j < P; ++j) {
+    const int op = t_.op[L_.start + j];
+    if (is_draw(op)) {
+      linear[j] = 1;
+      size[j] = 1.0;
+      continue;
     }
-    return kind == ARG_BODY && linear_form(ref, by, offset, draws);
-  };
-  const int ka = L_.kind_a[pos], ra = L_.ref_a[pos], kb = L_.kind_b[pos], rb = L_.ref_b[pos];
-  double v = 0;
-  switch (op) {
-    case NT_OP_NEG: return operand(ka, ra, -scale);
-    case NT_OP_ADD: return operand(ka, ra, scale) && operand(kb, rb, scale);
-    case NT_OP_SUB: return operand(ka, ra, scale) && operand(kb, rb, -scale);
-    case NT_OP_MUL:
-      if (literal(kb, rb, v)) return operand(ka, ra, scale * v);
-      return literal(ka, ra, v) && operand(kb, rb, scale * v);
-    case NT_OP_DIV: return literal(kb, rb, v) && operand(ka, ra, scale / v);
-    default: return false;
+    if (t_.active[L_.start + j]) continue;
+    const int ka = L_.kind_a[j], ra = L_.ref_a[j], kb = L_.kind_b[j], rb = L_.ref_b[j];
+    int terms = 0;
+    bool ok = true;
+    double by = 1.0;
+    auto term = [&](int kind, int ref) {
+      double v = 0;
+      if (kind == ARG_BODY && linear[ref]) {
+        size[j] += size[ref];
+        ++terms;
+      } else {
+        ok = ok && literal(kind, ref, v) && v == 0.0;
+      }
+    };
+    switch (op) {
+      case NT_OP_NEG: term(ka, ra); break;
+      case NT_OP_ADD:
+      case NT_OP_SUB:
+        term(ka, ra);
+        term(kb, rb);
+        break;
+      case NT_OP_MUL:
+        if (literal(kb, rb, by)) term(ka, ra);
+        else if (literal(ka, ra, by)) term(kb, rb);
+        else ok = false;
+        break;
+      case NT_OP_DIV:
+        ok = literal(kb, rb, by);
+        by = 1.0 / by;
+        if (ok) term(ka, ra);
+        break;
+      default: ok = false;
+    }
+    size[j] *= std::fabs(by);
+    linear[j] = ok && terms > 0 && std::isfinite(by) && std::isfinite(size[j]);
   }
+  return linear;
 }
 
 void Emitter::plan_draw_sums() {
@@ -2702,16 +2723,25 @@ void Emitter::plan_draw_sums() {
   after_.assign(P, 0);
   std::vector<char> sum(P, 0), draws(P, 0);
   int carries = 0;
+  bool any = false;
+  for (int j = 0; j < P; ++j) any |= j < static_cast<int>(gaff_.size()) && gaff_[j].on;
+  if (!any) return;
+  const std::vector<char> linear = linear_forms();
+  std::vector<char> form(P, 0);  // the forms and what they read
   for (int j = 0; j < P; ++j) {
-    if (!(j < static_cast<int>(gaff_.size()) && gaff_[j].on)) continue;
-    std::vector<char> own(P, 0);
-    double offset = 0;
-    if (!linear_form(gaff_[j].s_ref, 1.0, offset, own) || offset != 0.0) continue;
+    if (!(j < static_cast<int>(gaff_.size()) && gaff_[j].on) || !linear[gaff_[j].s_ref]) continue;
     sum[j] = 1;
     ++carries;
-    for (int d = 0; d < P; ++d) draws[d] |= own[d];
+    form[gaff_[j].s_ref] = 1;
   }
   if (!carries) return;
+  for (int j = P - 1; j >= 0; --j) {
+    if (!form[j]) continue;
+    const int ar = is_draw(t_.op[L_.start + j]) ? 0 : arity(t_.op[L_.start + j]);
+    draws[j] = ar == 0 && is_draw(t_.op[L_.start + j]);
+    if (ar >= 1 && L_.kind_a[j] == ARG_BODY) form[L_.ref_a[j]] = 1;
+    if (ar >= 2 && L_.kind_b[j] == ARG_BODY) form[L_.ref_b[j]] = 1;
+  }
   // nodes read by nothing but those exponents
   std::vector<std::vector<int>> users(P);
   std::vector<char> kept(P, 0), hoist(P, 0);

@@ -9,6 +9,8 @@ itself, a row that another value of the step reads, uniforms among the draws,
 and several markets."""
 from __future__ import annotations
 
+import time
+
 import numpy as np
 import pytest
 
@@ -36,6 +38,10 @@ def basket(nt, assets, draws, steps, form):
         extra = rec.constant(0.0)
         for _ in range(steps):
             z = [rec.randu() if form == "uniform" and d == 0 else rec.randn() for d in range(draws)]
+            if form.startswith("deep"):
+                # the first draw through a chain of sums that read one value twice
+                for _ in range(int(form[4:])):
+                    z[0] = z[0].add(z[0]).mul(0.5)
             rows = []
             for i in range(assets):
                 w = rec.constant(0.0)
@@ -59,7 +65,7 @@ def basket(nt, assets, draws, steps, form):
 
 
 CASES = [(3, 3, 16, "rows"), (3, 4, 17, "rows"), (4, 4, 15, "signed"), (5, 3, 40, "signed"), (4, 4, 33, "draw_read"),
-         (4, 4, 20, "row_read"), (4, 3, 31, "uniform"), (5, 5, 48, "rows")]
+         (4, 4, 20, "row_read"), (4, 3, 31, "uniform"), (5, 5, 48, "rows"), (4, 4, 18, "deep9")]
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
@@ -78,6 +84,18 @@ def test_draw_sums_match_the_oracle(nt, assets, draws, steps, form, precision):
         # fp32 rounding of the draws (2^-24 |z| each) through 48 steps at most, on spots of about 100
         ov, og = oracle.replay_paths(flat, 150, OFFSET, 42, f32=True, threads=1)
         assert rel_err(v, ov) < 2e-4 and rel_err(g, og) < 2e-3
+
+
+def test_a_deep_form_lowers_at_once(nt):
+    """Sums that read one value twice, 44 deep: each position of the step is
+    looked at once, where a walk along every way to the draw would take 2^44."""
+    from nablatensor_amd import rocm
+    for depth in (12, 22, 44):
+        flat = basket(nt, 5, 5, 16, f"deep{depth}")
+        started = time.monotonic()
+        src = rocm.lower(flat, rocm.options("fp64"))
+        assert time.monotonic() - started < 0.5, depth
+        assert "real ds" in src[:src.index("nt_replay_slow")]
 
 
 def test_draw_sums_shared_by_the_markets(nt):
