@@ -1336,9 +1336,9 @@ class Emitter {
   // Such an s that is a linear form of the step's draws with literal
   // coefficients (a correlated normal: a row of a Cholesky factor times the
   // step's normals): the form of the draws' sums is the sum of the forms, so
-  // the loop adds up the draws alone and the step's nodes that only feed such
-  // exponents (hoist_) are evaluated once, after the loop, on those sums
-  // (hoisted_step). For a worst-of basket of 16 assets that takes the 136 fma
+  // the loop adds up the draws alone, without the nodes that only feed such
+  // exponents (hoist_), and the forms are evaluated once, after the loop, on
+  // those sums (hoisted_step). For a worst-of basket of 16 assets that takes the 136 fma
   // of the step's 16 x 16 triangular map out of the loop: 2.55 -> 1.89 ms
   // (fp32) and 6.63 -> 5.02 ms (fp64) per 10^6 paths of 252 steps. Taken when
   // it saves at least kSumSaves instructions per step (the carries' sums and
@@ -1351,8 +1351,8 @@ class Emitter {
   static constexpr int kSumSaves = 4;
   static constexpr int kSumSteps = 16;
   // per loop position: a draw summed over the loop; a node the loop does not
-  // emit; a node evaluated after it (hoisted, or part of a form the step
-  // reads for something else too)
+  // emit; a node evaluated after it, on the sums (the forms and what they read,
+  // not the exponents that read the forms: those take S in geo_affine_finish)
   std::vector<char> dsum_, hoist_, after_;
   void plan_draw_sums();
   std::vector<char> linear_forms() const;
@@ -2764,7 +2764,6 @@ void Emitter::plan_draw_sums() {
   if (saved < kSumSaves) return;
   dsum_ = draws;
   hoist_ = hoist;
-  after_ = hoist;
   for (int j = 0; j < P; ++j) {
     if (!sum[j]) continue;
     gaff_[j].linear = true;
@@ -2808,8 +2807,8 @@ void Emitter::draw_sum(int U, int u, int j, std::map<std::pair<int, int>, std::s
   o_ << ind << own << " += " << z << ";\n";
 }
 
-// After the loop: the hoisted nodes of a step on the draws' sums, and each
-// carry's S = 0 + s of them.
+// After the loop: the step's linear forms on the draws' sums, and each carry's
+// S = 0 + s of them.
 void Emitter::hoisted_step() {
   const std::string ind = "    ";
   for (int j = 0; j < L_.period; ++j) {

@@ -9,6 +9,7 @@ itself, a row that another value of the step reads, uniforms among the draws,
 and several markets."""
 from __future__ import annotations
 
+import re
 import time
 
 import numpy as np
@@ -84,6 +85,19 @@ def test_draw_sums_match_the_oracle(nt, assets, draws, steps, form, precision):
         # fp32 rounding of the draws (2^-24 |z| each) through 48 steps at most, on spots of about 100
         ov, og = oracle.replay_paths(flat, 150, OFFSET, 42, f32=True, threads=1)
         assert rel_err(v, ov) < 2e-4 and rel_err(g, og) < 2e-3
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_only_the_forms_are_evaluated_on_the_sums(nt, precision):
+    """After the loop the step's form is taken on the draws' sums; the exponent and
+    the exponential it fed belong to one step and are not emitted on them."""
+    from nablatensor_amd import rocm
+    src = rocm.lower(basket(nt, 3, 3, 16, "rows"), rocm.options(precision, mode=2))
+    fast = src[:src.index("nt_replay_slow")]
+    after = fast[fast.index("real r0_", fast.index("}", fast.index("nt_normal_pair_sum"))):]
+    on_sums = [line for line in after.splitlines() if line.strip().startswith("const real r0_")]
+    assert len(on_sums) >= 6  # three sums, three rows or more
+    assert not [line for line in on_sums if "exp" in line or "in0" in line or re.search(r"\bv\d", line)], on_sums
 
 
 def test_a_deep_form_lowers_at_once(nt):
