@@ -8,6 +8,7 @@
 #include <dlfcn.h>
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
+#include <limits.h>
 #include <sys/stat.h>
 #include <utime.h>
 
@@ -152,15 +153,36 @@ std::vector<std::string> compile_options(const std::string& src, bool dump) {
 // every other use.
 thread_local std::string t_test_source_suffix;
 
+// The compiler this process has loaded: hipRTC's version, and the files of
+// hipRTC and of the comgr that compiles for it. A process that imported torch
+// first has torch's own pair, whose registers for one source differ from
+// ROCm's (the local-volatility sweep 338 and 336 VGPRs, the 252-step fp64 Asian
+// 80 and 94), so each keeps its own code objects.
+std::string compiler_id() {
+  int major = 0, minor = 0;
+  hiprtcVersion(&major, &minor);
+  std::string id = "hiprtc " + std::to_string(major) + "." + std::to_string(minor);
+  const void* symbols[] = {reinterpret_cast<const void*>(&hiprtcCompileProgram),
+                           reinterpret_cast<const void*>(&amd_comgr_do_action)};
+  for (const void* s : symbols) {
+    Dl_info info;
+    if (!dladdr(s, &info) || !info.dli_fname) continue;
+    char real[PATH_MAX];
+    const char* path = realpath(info.dli_fname, real) ? real : info.dli_fname;
+    struct stat st;
+    id += std::string(" ") + path + " " + std::to_string(stat(path, &st) == 0 ? static_cast<long long>(st.st_size) : 0);
+  }
+  return id;
+}
+
 int compile_hiprtc(const std::string& lowered, bool dump, std::vector<char>& code, double& seconds) {
   const std::string& src = t_test_source_suffix.empty() ? lowered : lowered + t_test_source_suffix;
   const auto t0 = std::chrono::steady_clock::now();
   const std::vector<std::string> opts = compile_options(src, dump);
-  int major = 0, minor = 0;
-  hiprtcVersion(&major, &minor);
   std::string key = src + "\n#opts";
   for (auto& o : opts) key += " " + o;
-  key += "\n#hiprtc " + std::to_string(major) + "." + std::to_string(minor) + "\n";
+  static const std::string compiler = compiler_id();
+  key += "\n#" + compiler + "\n";
   // The skeleton and its tables (150 KB) are hashed once per process: hashed
   // anew they were 0.2 ms of every executable's creation.
   static const uint64_t skeleton = fnv1a(NT_MATH_TABLES_SRC, fnv1a(NT_SKELETON_SRC));

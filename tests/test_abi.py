@@ -3,7 +3,10 @@ the lowering entry points and offline hipRTC compilation for gfx950."""
 from __future__ import annotations
 
 import ctypes as C
+import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -143,3 +146,30 @@ def test_spilling_kernel_is_declined(rocm, nt):
     assert rocm.compile_check(flat, rocm.options("fp64", mode=rocm.NT_MODE_REVERSE))["scratch_bytes"] == 0
     info = rocm.compile_check(flat, rocm.options("fp64", mode=rocm.NT_MODE_REVERSE, roll=-1))
     assert info["scratch_bytes"] == 0 and info["n_segments"] == 13 and info["checkpoint"] == rocm.NT_CKPT_RECOMPUTE
+
+
+def test_code_objects_are_kept_per_compiler(tmp_path):
+    """A process that has loaded torch compiles with torch's hipRTC and comgr,
+    another with ROCm's: their code objects for one source lie apart, and each
+    process reads its own."""
+    program = """
+import sys
+if "torch" in sys.argv: import torch
+import nablatensor_amd as nt
+from nablatensor_amd import rocm
+flat = nt.record(nt.Products.europeanCall(), nt.EquityMarket.atmOneYear(), nt.TimeGrid.uniform(1)).flat()
+info = rocm.compile_check(flat, rocm.options("fp64"))
+lib = sorted({line.split()[-1] for line in open("/proc/self/maps") if "libhiprtc.so" in line})
+print("RESULT", lib, info["vgprs"])
+"""
+    seen, entries = {}, []
+    for which in ("plain", "torch", "plain", "torch"):
+        env = dict(os.environ, NABLATENSOR_ROCM_CACHE=str(tmp_path), PYTHONPATH=str(ROOT))
+        run = subprocess.run([sys.executable, "-c", program, which], env=env, cwd=tmp_path, text=True,
+                             capture_output=True, timeout=300)
+        assert run.returncode == 0, run.stderr
+        result = run.stdout[run.stdout.index("RESULT"):]
+        assert seen.setdefault(which, result) == result  # the same compiler's object on the second run
+        entries.append(len(list(tmp_path.glob("*.co"))))
+    compilers = len({result.split("]")[0] for result in seen.values()})
+    assert entries == [1, compilers, compilers, compilers]
