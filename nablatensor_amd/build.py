@@ -123,16 +123,18 @@ def check_offline_hipcc(source: str, name: str = "check") -> Path:
 
 def build_math_device(force: bool = True) -> Path:
     """Test driver of the skeleton's own fp64 math on the device
-    (tests/device_math/nt_math_device.hip -> libnt_math_device.so, loaded by
+    (tests/device_math/nt_math_device.hip -> libnt_math_device.so and, with the
+    routines of NT_TURN_DRAWS, libnt_math_device_turn.so; loaded by
     tests/test_gpu_math.py)."""
     src = ROOT / "tests" / "device_math" / "nt_math_device.hip"
-    out = src.parent / "libnt_math_device.so"
     deps = [src, CSRC / "nt_skeleton.h", CSRC / "nt_math_tables.h"]
-    if not force and _newer(out, deps):
-        return out
-    _run([str(ROCM / "bin" / "hipcc"), "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
-          *PACKED_FP32_OFF, f"-I{CSRC}", str(src), "-o", str(out) + ".tmp"])
-    os.replace(str(out) + ".tmp", out)
+    for suffix, defines in (("_turn", ["-DNT_TURN_DRAWS=1"]), ("", [])):
+        out = src.parent / f"libnt_math_device{suffix}.so"
+        if not force and _newer(out, deps):
+            continue
+        _run([str(ROCM / "bin" / "hipcc"), "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+              *PACKED_FP32_OFF, *defines, f"-I{CSRC}", str(src), "-o", str(out) + ".tmp"])
+        os.replace(str(out) + ".tmp", out)
     return out
 
 

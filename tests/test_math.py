@@ -1,7 +1,8 @@
 """Accuracy of the skeleton's own fp64 log / sqrt / sincos / exp
 (nt_skeleton.h), built for the host, against mpmath at 40 digits; and of the
 Box-Muller pair against the oracle's glibc evaluation of the reference
-formula."""
+formula. Each test runs on the routines of most tapes and on those of tapes
+with the square root of an active drawn value (NT_TURN_DRAWS)."""
 from __future__ import annotations
 
 import ctypes as C
@@ -19,12 +20,19 @@ from conftest import ROOT
 
 mp.mp.dps = 40
 EMU = ROOT / "tests" / "host_emu"
+# Largest error of a sine or cosine in units of 2^-53 (the spacing of doubles in
+# [1/2, 1)). Rounding the final sum costs 0.5. The short routine adds the
+# roundings of its correction, which is at most pi/512 (three of 2^-61: 0.01),
+# and its table's errors (under 0.05 each by the choice of the angles): 0.58
+# measured. The other's table values are rounded (0.5 more): 1.04 measured.
+SINCOS_BOUND = {"short": 0.6, "turn": 1.1}
 
 
-@pytest.fixture(scope="module")
-def lib():
-    out = Path(tempfile.gettempdir()) / f"nt_math_emu_{os.getpid()}.so"  # one per test worker
-    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off", "-w",
+@pytest.fixture(scope="module", params=["short", "turn"])
+def lib(request):
+    out = Path(tempfile.gettempdir()) / f"nt_math_emu_{request.param}_{os.getpid()}.so"  # one per test worker
+    turn = ["-DNT_TURN_DRAWS=1"] if request.param == "turn" else []
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off", "-w", *turn,
                     f"-I{ROOT / 'nablatensor_amd' / 'csrc'}", f"-I{EMU}", str(EMU / "math_main.cpp"),
                     "-o", str(out)], check=True)
     L = C.CDLL(str(out))
@@ -37,6 +45,7 @@ def lib():
     L.emu_sqrt_q.argtypes = [P(C.c_double), P(C.c_double), P(C.c_double), P(C.c_int), C.c_long]
     L.emu_recip.argtypes = [P(C.c_double), P(C.c_double), P(C.c_int), C.c_long]
     L.emu_normal_pair.argtypes = [P(C.c_uint32)] * 3 + [P(C.c_double)] * 2 + [C.c_long]
+    L.sincos_bound = SINCOS_BOUND[request.param]
     return L
 
 
@@ -124,7 +133,7 @@ def test_sincos_within_two_ulp(lib):
         # error relative to the unit circle scale: sin near 0 is judged in absolute terms
         worst = max(worst, float(abs(mp.mpf(si) - mp.sin(th)) / mp.mpf(2.0**-53)),
                     float(abs(mp.mpf(cj) - mp.cos(th)) / mp.mpf(2.0**-53)))
-    assert worst <= 2.0, worst
+    assert worst <= lib.sincos_bound, worst
 
 
 def test_sqrt_within_one_ulp(lib):
