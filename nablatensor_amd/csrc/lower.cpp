@@ -3291,7 +3291,7 @@ void Emitter::kernel_head(bool slow) {
   o_ << "  const nt_u64 nt_words = T >> 6;  // lane bitmap words per market\n";
   o_ << "  nt_u64* __restrict__ nt_bits = flags + 1;\n";
   o_ << "  (void)scratch; (void)out_v; (void)out_g; (void)nt_bits; (void)nt_words;\n";
-  if (!slow) o_ << "#ifdef NT_ROWS\n  const nt_u64 nt_t0 = nt_clock();\n#endif\n";
+  if (!slow && M == 1) o_ << "#ifdef NT_ROWS\n  const nt_u64 nt_t0 = nt_clock();\n#endif\n";
   const int nacc = p_.n_channels * M;
   o_ << "  double acc[" << nacc << "];\n";
   o_ << "  for (int c = 0; c < " << nacc << "; ++c) acc[c] = 0.0;\n";
@@ -3755,15 +3755,15 @@ void Emitter::kernel(bool slow) {
     o_ << ") atomicAdd(flags, 1ull);\n";
   }
   const int nacc = p_.n_channels * M;
-  o_ << "  __shared__ double nt_lds[" << nacc << " * (" << p_.block << " / 64)];\n";
-  if (!slow) {
-    // a small dispatch's blocks write their sums for the host to add
-    std::string bad = "false";
-    for (int m = 0; m < M && fb; ++m) bad = (m ? bad + " || " : std::string()) + "nt_lane_bad" + std::to_string(m);
-    o_ << "#ifdef NT_ROWS\n  nt_block_out<" << nacc << ">(acc, partials, nt_lds, out_v, " << bad << ", nt_t0);\n#else\n";
+  // a small dispatch's blocks write their sums for the host to add, and whether they left paths
+  const bool rows = !slow && M == 1;
+  o_ << "  __shared__ double nt_lds[" << nacc + (rows ? 1 : 0) << " * (" << p_.block << " / 64)];\n";
+  if (rows) {
+    o_ << "#ifdef NT_ROWS\n  nt_block_out<" << nacc << ">(acc, partials, nt_lds, out_v, " << (fb ? "nt_lane_bad0" : "false")
+       << ", nt_t0);\n#else\n";
   }
   o_ << "  nt_block_store<" << nacc << ">(acc, partials, nt_lds);\n";
-  if (!slow) o_ << "#endif\n";
+  if (rows) o_ << "#endif\n";
   o_ << "}\n";
   slow_ = false;
   mlo_ = 0;

@@ -618,7 +618,10 @@ __device__ __forceinline__ void nt_block_store(const double (&acc)[NCH], double*
 // by one while the kernel ends: each is then a store of its own to system
 // scope. Otherwise the host reads them after the kernel's end, and a wave's
 // plain stores leave as whole lines (391 blocks of 9 words: 97 us per weekday
-// Asian dispatch against 102).
+// Asian dispatch against 102). The waves' bad lanes meet through `lds`, which
+// holds (NCH + 1) * (blockDim.x / 64) doubles: a __syncthreads_or (256 bytes
+// of LDS and its own reduction) took the fp32 Heston kernel from 80 to 86
+// VGPRs, six waves to five.
 #ifndef NT_DUMP_PATHS
 #define NT_ROWS 1
 #endif
@@ -639,7 +642,9 @@ __device__ __forceinline__ void nt_block_out(const double (&acc)[NCH], double* _
     const double w = nt_wave_sum(acc[c]);
     if (lane == 0) lds[c * waves + wave] = w;
   }
-  const nt_u64 any = __syncthreads_or(bad) ? 1 : 0;
+  const nt_u64 bad_lanes = __ballot(bad);
+  if (lane == 0) lds[NCH * waves + wave] = bad_lanes != 0 ? 1.0 : 0.0;
+  __syncthreads();
   const bool watched = (reinterpret_cast<nt_u64>(rows) & 1) != 0;
   double* row = reinterpret_cast<double*>(reinterpret_cast<nt_u64>(rows) & ~1ull) +
                 static_cast<nt_u64>(blockIdx.x) * (NCH + 2);
@@ -651,8 +656,10 @@ __device__ __forceinline__ void nt_block_out(const double (&acc)[NCH], double* _
     if (rows) nt_to_host(row + 2 + c, s, watched);
   }
   if (rows && threadIdx.x == 0) {
+    double any = 0.0;
+    for (int w = 0; w < waves; ++w) any += lds[NCH * waves + w];
     nt_to_host(reinterpret_cast<nt_u64*>(row), started, watched);
-    nt_to_host(reinterpret_cast<nt_u64*>(row) + 1, (nt_clock() << 1) | any, watched);
+    nt_to_host(reinterpret_cast<nt_u64*>(row) + 1, (nt_clock() << 1) | (any > 0.0 ? 1 : 0), watched);
   }
 }
 

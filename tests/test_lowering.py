@@ -949,3 +949,14 @@ def test_special_values_follow_the_oracle_emulated(nt, rocm, mode):
                 # the reverse sweep's adjoints, special values included (tangent mode caps sqrt's
                 # infinite derivative at 0 and can differ in the sign of a zero derivative)
                 assert close_special(np.reshape(g, og.shape), og, 4e-16), (case, flat["output_node"], g[:1], og[:1])
+
+
+def test_the_rows_of_small_dispatches_cost_no_wave(rocm, tapes):
+    """The epilogue that can leave a block's sums to the host is in every replay
+    kernel: fp32 kernels at the edge of a wave keep it (512 registers a SIMD lane:
+    80 are six waves, 64 are eight). Kernels of several markets have none of it."""
+    from nablatensor_amd import workloads
+    assert rocm.compile_check(tapes["C4"], rocm.options("fp32"))["vgprs"] <= 80
+    assert rocm.compile_check(workloads.local_vol_asian_tape(2, 252).flat(), rocm.options("fp32"))["vgprs"] <= 64
+    one, many = (rocm.lower(tapes["C2"], rocm.options("fp64", markets=m)) for m in (1, 3))
+    assert "nt_block_out" in one and "nt_block_out" not in many and "nt_clock" not in many
