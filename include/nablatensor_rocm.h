@@ -181,7 +181,9 @@ int nt_exec_set_inputs(nt_exec *exec, const double *inputs, int32_t n);
  * stream (a dispatch on few blocks, 512 at most, has no finishing kernel: the host
  * adds the blocks' sums, in the same order, and kernel_ms is the replay
  * kernel's time by the device's clock, from its first block's start to its
- * last block's end), wall_ms from entry to sums on the host. Replaces
+ * last block's end; on 128 blocks or fewer the call may return once the sums are in,
+ * before the runtime has seen the kernel's end, which every 256th such call
+ * waits for, so an error found there comes from a later call), wall_ms from entry to sums on the host. Replaces
  * DeviceAadExecutable.replay (DeviceAadExecutable.java:139-168), returning raw
  * sums instead of means so callers can combine dispatches exactly. */
 int nt_exec_replay(nt_exec *exec, uint64_t paths, uint64_t offset, uint64_t seed,

@@ -64,6 +64,7 @@ constexpr size_t kRowWords = 4608;  // most words of their rows (rows_fit)
 constexpr size_t kRowChannels = 128;  // and most sums of one (the host adds 64 lanes of them)
 constexpr int kWatchBlocks = 128;  // most blocks whose rows the host watches for, and for how long (await_rows)
 constexpr int kWatchMicros = 1000;
+constexpr int kUndrained = 256;  // a stream is waited for at least once in so many watched dispatches
 constexpr uint64_t kUnwritten = 0x7ff5a3c96e1d2b47ull;  // a signalling NaN that no arithmetic gives
 
 // ---- code-object cache ---------------------------------------------------------
@@ -501,6 +502,12 @@ size_t flags_bytes_for(uint64_t lanes, int markets) {
   return (1 + static_cast<size_t>((lanes + 63) / 64) * static_cast<size_t>(std::max(1, markets))) * sizeof(uint64_t);
 }
 
+static int drain(nt_exec* x) {
+  NT_HIP(hipStreamSynchronize(x->stream), "hipStreamSynchronize");
+  x->undrained = 0;
+  return NT_OK;
+}
+
 // A dispatch on at most kRowBlocks blocks, with at most kRowWords words of
 // rows, writes its blocks' sums to pinned host memory and the host adds them:
 // one launch and one wait, where the finishing pass costs a second launch, its
@@ -522,18 +529,21 @@ bool rows_fit(const nt_exec* x, int grid) {
 // 40 blocks 16.3 and 13.0 us, 79 blocks 24.2 and 22.2, 391 blocks 18.2 and
 // 20.1 (the European call and the 64-fixing Asian). After that (a long kernel,
 // a failed one, a sum that is that very NaN) the stream is drained as usual.
+// It is also drained every kUndrained dispatches, so that a run of small ones
+// leaves the runtime no more than that many to retire (a wait of about 6 us
+// in 256 dispatches of 11 to 22).
 int await_rows(nt_exec* x, int grid) {
   const size_t words = static_cast<size_t>(grid) * (static_cast<size_t>(x->low.plan.n_channels) + 2);
   const auto t0 = std::chrono::steady_clock::now();
   size_t w = grid <= kWatchBlocks ? 0 : words + 1;
   for (unsigned spins = 1; w <= words; ++spins) {
     while (w < words && __atomic_load_n(x->h_rows + w, __ATOMIC_ACQUIRE) != kUnwritten) ++w;
-    if (w == words) return NT_OK;
+    if (w == words && ++x->undrained < kUndrained) return NT_OK;
+    if (w == words) break;
     if ((spins & 63) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(kWatchMicros)) break;
     __builtin_ia32_pause();
   }
-  NT_HIP(hipStreamSynchronize(x->stream), "hipStreamSynchronize");
-  return NT_OK;
+  return drain(x);
 }
 
 // The sums of a small dispatch from its blocks' rows, in nt_finish's order:
@@ -616,6 +626,8 @@ extern "C" {
 int nt_abi_version(void) { return NT_ABI_VERSION; }
 
 void nt_testing_append_source(const char* text) { t_test_source_suffix = text ? text : ""; }
+
+int32_t nt_testing_undrained(const nt_exec* x) { return x ? x->undrained : 0; }
 
 const char* nt_last_error(void) { return ntr::last_error(); }
 
@@ -854,7 +866,8 @@ static int replay_rows(nt_exec* x, int grid, uint64_t paths, uint64_t offset, ui
     rc = launch_finish(x, x->fn_finish, x->fn_slow, x->d_partials, grid, nch, x->h_sums);
     if (rc != NT_OK) return rc;
     NT_HIP(hipEventRecord(x->ev[2], x->stream), "hipEventRecord");
-    NT_HIP(hipStreamSynchronize(x->stream), "hipStreamSynchronize");
+    rc = ntr::drain(x);
+    if (rc != NT_OK) return rc;
     NT_HIP(hipEventElapsedTime(&rest_ms, x->ev[0], x->ev[2]), "hipEventElapsedTime");
     std::memcpy(sums, x->h_sums, sizeof(double) * nch);
   }
@@ -894,7 +907,8 @@ int nt_exec_replay(nt_exec* x, uint64_t paths, uint64_t offset, uint64_t seed, d
   }
   if (rc != NT_OK) return rc;
   NT_HIP(hipEventRecord(x->ev[2], x->stream), "hipEventRecord");
-  NT_HIP(hipStreamSynchronize(x->stream), "hipStreamSynchronize");
+  rc = ntr::drain(x);
+  if (rc != NT_OK) return rc;
   if (x->fn_slow && *x->h_deferred != 0) {
     rc = ntr::launch_slow_on(x, x->stream, x->fn_slow, x->d_inputs, x->d_partials, nch, x->d_scratch, x->d_flags,
                              paths, offset, seed, nullptr, nullptr, grid);
@@ -1062,7 +1076,8 @@ int nt_exec_replay_many(nt_exec* x, const double* input_sets, int32_t markets, u
     }
     NT_HIP(hipEventRecord(x->ev[2], x->stream), "hipEventRecord");
   }
-  NT_HIP(hipStreamSynchronize(x->stream), "hipStreamSynchronize");
+  const int drained = ntr::drain(x);
+  if (drained != NT_OK) return drained;
   std::memcpy(sums, x->h_sums, sizeof(double) * need);
   if (timing) {
     float ms = 0;

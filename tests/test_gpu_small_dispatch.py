@@ -91,3 +91,24 @@ def test_inputs_changed_between_small_and_large_dispatches(nt, rocm):
             x.set_inputs(sets[m])
             assert np.array_equal(x.replay(n, 0, 9)[0], want[n][m]), (m, n)
             assert np.array_equal(x.replay(1_000, 0, 9)[0], want[1_000][m]), (m, n)
+
+
+def test_watched_dispatches_are_drained(nt, rocm):
+    """A dispatch whose rows the host watches for returns without waiting for the
+    stream, at most 255 times running; any other dispatch waits for it."""
+    import ctypes as C
+    undrained = rocm.lib().nt_testing_undrained
+    undrained.argtypes, undrained.restype = [C.c_void_p], C.c_int32
+    with rocm.Executable(tape_of(nt, "european"), rocm.options("fp64")) as x:
+        seen = []
+        print("case 600 watched dispatches", flush=True)
+        for k in range(600):
+            x.replay(1_000, k * 1_000, 5)
+            seen.append(undrained(x._h))
+        # one more each time, zero after 255 or where the sums took longer than the host watches
+        assert all(b == (a + 1 if a < 255 else 0) or b == 0 for a, b in zip(seen, seen[1:])) and max(seen) <= 255
+        x.replay(200 * 256, 0, 5)  # too many blocks to watch for
+        assert undrained(x._h) == 0
+        x.replay(1_000, 0, 5)
+        x.replay(600 * 256, 0, 5)  # the finishing kernel adds these
+        assert undrained(x._h) == 0
