@@ -1125,10 +1125,12 @@ class Emitter {
         break;
       case NT_OP_DIV:
         if (rev_fused_) {
+          // the quotient before the reciprocal: adjoint / divisor alone may be
+          // subnormal (or overflow) where adjoint * quotient / divisor is not
           const std::string q = "q" + Ai;
-          o_ << ind << "const real " << q << " = " << Ai << " * nt_recip(" << Vb << ", nt_slow);\n";
-          add(Aa, q);
-          add(Ab, q + " * " + Vi, true);
+          o_ << ind << "const real " << q << " = nt_recip(" << Vb << ", nt_slow);\n";
+          add(Aa, Ai + " * " + q);
+          add(Ab, Ai + " * " + Vi + " * " + q, true);
           break;
         }
         add(Aa, Ai + " / " + Vb);

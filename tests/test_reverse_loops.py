@@ -76,6 +76,27 @@ def test_reverse_rules_match_the_oracle(nt, kind, size, steps, ckpt, precision):
         assert rel_err(v, ov) < 2e-4 and rel_err(g, og) < 2e-3
 
 
+def test_quotients_of_far_apart_sizes(nt):
+    """A divisor's adjoint where adjoint / divisor (1e-313) is subnormal and
+    adjoint * quotient / divisor (1e-36) is not."""
+    from nablatensor_amd import rocm
+
+    def body(rec):
+        x, s = rec.input("a", 1e23), rec.constant(0.0)
+        for _ in range(16):
+            s = s.add(rec.constant(1e300).div(x).mul(1e-290).mul(rec.randn()))
+            x = x.mul(1.001)
+        rec.output(s)
+
+    flat = nt.AadRecorder.record(body).flat()
+    src = rocm.lower(flat, rocm.options("fp64", mode=1))
+    assert "nt_recip" in src
+    _, v, g = emu.EmulatedKernel(src, 1, tape_slots(src)).run(flat["recorded_inputs"], 50, 0, 42, grid=1, block=64)
+    ov, og = oracle.replay_paths(flat, 50, 0, 42, threads=1)
+    # 16 steps of four roundings each, whose sum may cancel a few digits
+    assert np.abs(v / ov - 1.0).max() < 1e-13 and np.abs(g / og - 1.0).max() < 1e-13
+
+
 def test_variance_roots_keep_their_rounding(nt, tapes):
     """A tape with the square root of an active drawn value is not contracted."""
     from nablatensor_amd import rocm
