@@ -2263,8 +2263,6 @@ void Emitter::body_tangent_operand(int u, int kind, int ref, std::function<std::
   }
 }
 
-// One trip of U loop iterations: values and their tangents, then the carried
-// state (values and tangents) advances.
 // Value of loop position j in iteration u of the trip, from its operands x
 // and y, for what needs no statement of its own before it.
 std::string Emitter::body_rhs(int u, int j, const std::string& x, const std::string& y) const {
@@ -2289,6 +2287,8 @@ std::string Emitter::body_rhs(int u, int j, const std::string& x, const std::str
   return body_expr(j, u, op, x, y);
 }
 
+// One trip of U loop iterations: values and their tangents, then the carried
+// state (values and tangents) advances.
 void Emitter::tsegment(int U, const std::string& sg) {
   const int P = L_.period, s = L_.start;
   const std::string ind = "      ";

@@ -64,7 +64,7 @@ struct nt_exec {
   double* h_grown = nullptr;       // their own allocation once several input sets outgrow the first
   uint32_t* h_deferred = nullptr;  // pinned host word: the finishing pass found flagged lanes (nt_exec_replay)
   double* h_inputs = nullptr;      // inputs of a small dispatch, read by its kernel from here
-  uint64_t* h_rows = nullptr;      // the blocks' sums of a small dispatch (nt_block_rows)
+  uint64_t* h_rows = nullptr;      // the blocks' sums of a small dispatch (the skeleton's nt_block_out)
   std::vector<double> lane_sums;   // scratch of the host's finishing pass
   double clock_khz = 0;            // rate of the device clock in the rows
   int undrained = 0;               // watched dispatches since the stream was last waited for (await_rows)

@@ -59,7 +59,7 @@ using ntr::MarketVariant;
 namespace {
 
 const char* kArch = "gfx950";
-constexpr int kRowBlocks = 512;    // most blocks whose sums the host adds (finish_rows)
+constexpr int kRowBlocks = 512;    // most blocks whose sums the host adds: eight for each of 64 lanes (finish_rows)
 constexpr size_t kRowWords = 4608;  // most words of their rows (rows_fit)
 constexpr size_t kRowChannels = 128;  // and most sums of one (the host adds 64 lanes of them)
 constexpr int kWatchBlocks = 128;  // most blocks whose rows the host watches for, and for how long (await_rows)
@@ -547,9 +547,8 @@ int await_rows(nt_exec* x, int grid) {
 }
 
 // The sums of a small dispatch from its blocks' rows, in nt_finish's order:
-// lane l of 64 adds the blocks 8 (l + 64 k) + x, x = 0..7 the outer loop and k
-// the inner (kRowBlocks is within one batch of the pass), and the lanes are
-// added by the wave's butterfly. Returns whether a block had a lane with paths
+// lane l of 64 adds the blocks 8 l + x, x = 0..7 (kRowBlocks is 8 x 64), and the
+// lanes are added by the wave's butterfly. Returns whether a block had a lane with paths
 // for the exception kernel; `ms` is the time from the first block's start to
 // the last block's end on the device clock.
 bool finish_rows(nt_exec* x, int grid, double* sums, double& ms) {
@@ -558,13 +557,13 @@ bool finish_rows(nt_exec* x, int grid, double* sums, double& ms) {
   std::fill_n(lane, static_cast<size_t>(64) * nch, 0.0);
   uint64_t first = ~0ull, last = 0, bad = 0;
   for (int cls = 0; cls < 8; ++cls) {
-    for (int b = cls; b < grid; b += 8) {  // k = b / 512 ascends within a lane
+    for (int b = cls; b < grid; b += 8) {
       const uint64_t* row = x->h_rows + static_cast<size_t>(b) * stride;
       first = std::min(first, row[0]);
       last = std::max(last, row[1] >> 1);
       bad |= row[1] & 1;
       const double* v = reinterpret_cast<const double*>(row + 2);
-      double* to = lane + static_cast<size_t>((b >> 3) & 63) * nch;
+      double* to = lane + static_cast<size_t>(b >> 3) * nch;
       for (int c = 0; c < nch; ++c) to[c] += v[c];
     }
   }
