@@ -344,11 +344,17 @@ int decline_spill(const nt_exec_info& info, const nt_options* opt) {
 
 // Compiles the lowered replay kernel. A kernel at one wave per SIMD cannot
 // hide the latency of its own dependent fp64 instructions (the VALU issues on
-// about half the cycles); one that needs at most 16 VGPRs more than two waves
-// allow (256) is compiled again with launch bounds asking for two, and that
-// code is kept when it fits without scratch (the 16-asset worst-of in fp64:
-// 270 VGPRs, one wave, 9.07 ms; 254 VGPRs, two waves, 7.12 ms). An explicit
-// nt_options.waves is left as asked.
+// about half the cycles); one that needs a few VGPRs more than two waves allow
+// (256) is compiled again with launch bounds asking for two, and that code is
+// kept when it fits without scratch (the 16-asset worst-of in fp64, when it
+// needed 270 VGPRs: one wave 9.07 ms, two 7.12 ms). A few: 16 for a reverse
+// sweep, whose state at once is what it needs (the local-volatility Asian at 17
+// and 18 coefficients, 266 and 276 VGPRs, spills 52 and 92 bytes when asked for
+// two waves); 32 in tangent mode, where the code after the loop then holds one
+// asset's values at a time (worst-ofs of 12 and 15 assets, 3x10^5 paths of 252
+// steps: 273 and 276 VGPRs, one wave, 1.24 and 2.25 ms; 158 and 195 VGPRs, 1.05
+// and 1.50 ms). An explicit nt_options.waves is left as asked.
+constexpr int kSecondWaveReverse = 16, kSecondWaveTangent = 32;
 int compile_replay(const nt_tape* tape, const nt_options* options, Lowered& low, std::vector<char>& code,
                    nt_exec_info& info) {
   double secs = 0;
@@ -358,7 +364,8 @@ int compile_replay(const nt_tape* tape, const nt_options* options, Lowered& low,
   kernel_resources(code, "nt_replay", info);
   info.compile_seconds = secs;
   const bool asked = options && options->waves > 0;
-  if (asked || info.vgprs <= 256 || info.vgprs > 256 + 16) return NT_OK;
+  const int over = low.plan.mode == NT_MODE_TANGENT ? kSecondWaveTangent : kSecondWaveReverse;
+  if (asked || info.vgprs <= 256 || info.vgprs > 256 + over) return NT_OK;
   nt_options o = options ? *options : nt_options{};
   o.waves = 2;
   Lowered low2;

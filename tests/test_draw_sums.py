@@ -1,7 +1,7 @@
 """A step's linear map of its draws, taken once on the draws' sums after the
 loop: baskets of GBM spots read only by the payoff, whose step exponents take
-correlated normals (rows of a literal matrix), compiled for the host and held
-to the oracle per path. Cases: three to five assets (three is the smallest
+correlated normals (rows of a literal matrix), compiled for the host and on the
+device, held to the oracle per path. Cases: three to five assets (three is the smallest
 basket that takes it), an odd number of draws per step (Box-Muller pairs split
 over two steps), step counts around the fp32 sums' 16 steps, rows written as
 differences, a draw that the step also reads by
@@ -125,3 +125,25 @@ def test_draw_sums_shared_by_the_markets(nt):
     for m in range(3):
         s1, v1, g1 = emu.EmulatedKernel(one, len(x0), 0).run(sets[m], 120, OFFSET, 7, grid=2, block=64)
         assert np.array_equal(v[m], v1) and np.array_equal(g[m], g1) and np.array_equal(sums[m], s1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("assets,draws,steps,form", CASES + [(12, 12, 17, "rows"), (7, 6, 16, "signed")])
+def test_draw_sums_on_the_device(nt, assets, draws, steps, form, precision):
+    from nablatensor_amd import rocm
+    flat = basket(nt, assets, draws, steps, form)
+    print(f"case {form} assets={assets} draws={draws} steps={steps} {precision}", flush=True)
+    with rocm.Executable(flat, rocm.options(precision, mode=2)) as x:
+        assert "real ds" in x.source()
+        for paths in (1, 257, 3_000):
+            v, g = x.replay_paths(paths, OFFSET, 42)
+            sums, _ = x.replay(paths, OFFSET, 42)
+            if precision == "fp64":
+                check_per_path(v, g, flat, paths, OFFSET, 42, min_strict=0.0 if paths == 1 else 0.9)
+            else:  # the emulator test's bounds, on the same tapes
+                ov, og = oracle.replay_paths(flat, paths, OFFSET, 42, f32=True, threads=1)
+                assert rel_err(v, ov) < 2e-4 and rel_err(g, og) < 2e-3
+            rows = np.concatenate([v.reshape(-1, 1), v.reshape(-1, 1) ** 2, g.reshape(paths, -1)], axis=1)
+            # the sums of the same rows in another order: 3,000 roundings at most, 1.1e-16 each
+            assert np.all(np.abs(sums - rows.sum(0)) <= 1e-12 * np.maximum(np.abs(rows).sum(0), 1e-300))

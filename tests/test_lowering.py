@@ -960,3 +960,14 @@ def test_the_rows_of_small_dispatches_cost_no_wave(rocm, tapes):
     assert rocm.compile_check(workloads.local_vol_asian_tape(2, 252).flat(), rocm.options("fp32"))["vgprs"] <= 64
     one, many = (rocm.lower(tapes["C2"], rocm.options("fp64", markets=m)) for m in (1, 3))
     assert "nt_block_out" in one and "nt_block_out" not in many and "nt_clock" not in many
+
+
+@pytest.mark.parametrize("assets", [12, 15, 16])
+def test_wide_baskets_hold_two_waves(nt, rocm, assets):
+    """fp64 worst-of kernels, whose first compile may need up to 276 VGPRs: at most 256, no scratch."""
+    from nablatensor_amd import workloads
+    fx = workloads.worst_of_inputs()
+    basket = nt.WorstOfBasket.call([row[:assets] for row in fx["corr"][:assets]], 100.0, 1.0, 252)
+    flat = nt.record(basket, nt.WorstOfBasket.market([100.0] * assets, fx["sigma"][:assets], 0.03)).flat()
+    info = rocm.compile_check(flat, rocm.options("fp64"))
+    assert info["vgprs"] <= 256 and info["scratch_bytes"] == 0
