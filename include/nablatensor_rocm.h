@@ -178,12 +178,12 @@ int nt_exec_set_inputs(nt_exec *exec, const double *inputs, int32_t n);
  * when built price-only), the AadTotals fields (AadTotals.java:30-40); n_sums
  * must be n_outputs * (2 + n_inputs). timing (nullable) receives {kernel_ms, wall_ms}: kernel_ms from
  * HIP events around the replay and finishing kernels on the executable's
- * stream (a dispatch on few blocks, 512 at most, has no finishing kernel: the host
- * adds the blocks' sums, in the same order, and kernel_ms is the replay
- * kernel's time by the device's clock, from its first block's start to its
- * last block's end; on 128 blocks or fewer the call may return once the sums are in,
- * before the runtime has seen the kernel's end, which every 256th such call
- * waits for, so an error found there comes from a later call), wall_ms from entry to sums on the host. Replaces
+ * stream, wall_ms from entry to sums on the host. A dispatch on few blocks (512 at
+ * most) has no finishing kernel: the host adds the blocks' sums, in the same
+ * order, and kernel_ms is the replay kernel's time by the device's clock, from
+ * its first block's start to its last block's end. Such a call may return once
+ * the sums are in, before the runtime has seen the kernel's end, which every
+ * 256th of them waits for; an error found there comes from a later call. Replaces
  * DeviceAadExecutable.replay (DeviceAadExecutable.java:139-168), returning raw
  * sums instead of means so callers can combine dispatches exactly. */
 int nt_exec_replay(nt_exec *exec, uint64_t paths, uint64_t offset, uint64_t seed,

@@ -67,7 +67,7 @@ struct nt_exec {
   uint64_t* h_rows = nullptr;      // the blocks' sums of a small dispatch (the skeleton's nt_block_out)
   std::vector<double> lane_sums;   // scratch of the host's finishing pass
   double clock_khz = 0;            // rate of the device clock in the rows
-  int undrained = 0;               // watched dispatches since the stream was last waited for (await_rows)
+  int undrained = 0;               // dispatches since the stream was last waited for (await_rows)
   size_t h_cap = 0;          // doubles in h_sums
   void* d_scratch = nullptr;
   size_t scratch_bytes = 0;  // bytes of d_scratch: the reverse sweep's per-lane tape at the resident grid

@@ -62,9 +62,8 @@ const char* kArch = "gfx950";
 constexpr int kRowBlocks = 512;    // most blocks whose sums the host adds: eight for each of 64 lanes (finish_rows)
 constexpr size_t kRowWords = 4608;  // most words of their rows (rows_fit)
 constexpr size_t kRowChannels = 128;  // and most sums of one (the host adds 64 lanes of them)
-constexpr int kWatchBlocks = 128;  // most blocks whose rows the host watches for, and for how long (await_rows)
-constexpr int kWatchMicros = 1000;
-constexpr int kUndrained = 256;  // a stream is waited for at least once in so many watched dispatches
+constexpr int kWatchMicros = 1000;  // how long the host watches for the rows (await_rows)
+constexpr int kUndrained = 256;     // the stream is drained at least once in so many such dispatches
 constexpr uint64_t kUnwritten = 0x7ff5a3c96e1d2b47ull;  // a signalling NaN that no arithmetic gives
 
 // ---- code-object cache ---------------------------------------------------------
@@ -517,36 +516,41 @@ static int drain(nt_exec* x) {
 
 // A dispatch on at most kRowBlocks blocks, with at most kRowWords words of
 // rows, writes its blocks' sums to pinned host memory and the host adds them:
-// one launch and one wait, where the finishing pass costs a second launch, its
-// wait for the replay kernel, its own 6 us and the three events that time the
-// two. Measured per dispatch, European call (9 words a block): 1 block 21.2 ->
-// 11 us, 40 blocks 22.7 -> 13.0, 391 blocks 23.6 -> 18.2; 768 blocks (6,912
-// words) 27.2 -> 30.8, where the host's reading of the rows and the blocks'
-// writes over PCIe cost more than the pass, as on a worst-of's 347 blocks of
-// 19 words (6,593): 35.9 -> 37.0 us.
+// one launch and no wait for the kernel's end, where the finishing pass costs a
+// second launch, its wait for the replay kernel, its own 6 us and the three
+// events that time the two. The pass against the rows, the same replay
+// kernels, us per dispatch: European call of 512 blocks of 9 words 25.9 and
+// 21.6 (fp32), 26.8 and 23.2 (fp64); 48-step Heston, 384 of 12, 41.2 and 33.3,
+// 58.9 and 50.8; worst-of of 4, 354 of 13, 38.7 and 30.4, 58.8 and 50.6; of
+// 16, 124 of 37, 60.8 and 51.9, 100.3 and 90.8. The limits are what 37 KB of
+// pinned memory per executable hold; the finishing pass's order gives each of
+// 64 lanes eight blocks there.
 bool rows_fit(const nt_exec* x, int grid) {
   const size_t nch = static_cast<size_t>(x->low.plan.n_channels);
   return nch <= kRowChannels && grid <= kRowBlocks && static_cast<size_t>(grid) * (nch + 2) <= kRowWords;
 }
 
-// Waits for the rows of a dispatch on at most kWatchBlocks blocks. Every word
-// was set to kUnwritten before the launch; the first kWatchMicros the host
-// watches for the words themselves, which arrive before the runtime sees the
-// kernel's end. Measured per dispatch, draining the stream against watching:
-// 40 blocks 16.3 and 13.0 us, 79 blocks 24.2 and 22.2, 391 blocks 18.2 and
-// 20.1 (the European call and the 64-fixing Asian). After that (a long kernel,
-// a failed one, a sum that is that very NaN) the stream is drained as usual.
-// It is also drained every kUndrained dispatches, so that a run of small ones
-// leaves the runtime no more than that many to retire (a wait of about 6 us
-// in 256 dispatches of 11 to 22).
+// Waits for the rows of a dispatch. Every word was set to kUnwritten before the
+// launch; the first kWatchMicros the host watches for the words themselves,
+// which arrive before the runtime sees the kernel's end. Draining the stream
+// instead against watching, us per dispatch: European 129 blocks 20.5 and
+// 16.6, 391 blocks 23.6 and 20.6 (fp32); 64-fixing Asian, 391 blocks, 38.3 and
+// 32.2, 252 weekday fixings, 391 blocks, 101.6 and 95.1, 504-step Heston, 352
+// blocks, 354.2 and 343.8 (fp64). (Drained, rows of over 3,950 words took up to
+// 1 us longer than the pass.) After kWatchMicros (a long kernel, a failed one, a sum that
+// is that very NaN) the stream is drained as usual. It is also drained every
+// kUndrained dispatches, so that a run of small ones leaves the runtime no more
+// than that many to retire (a wait of about 6 us in 256 dispatches of 11 to 22).
 int await_rows(nt_exec* x, int grid) {
   const size_t words = static_cast<size_t>(grid) * (static_cast<size_t>(x->low.plan.n_channels) + 2);
   const auto t0 = std::chrono::steady_clock::now();
-  size_t w = grid <= kWatchBlocks ? 0 : words + 1;
-  for (unsigned spins = 1; w <= words; ++spins) {
+  size_t w = 0;
+  for (unsigned spins = 1; ; ++spins) {
     while (w < words && __atomic_load_n(x->h_rows + w, __ATOMIC_ACQUIRE) != kUnwritten) ++w;
-    if (w == words && ++x->undrained < kUndrained) return NT_OK;
-    if (w == words) break;
+    if (w == words) {
+      if (++x->undrained < kUndrained) return NT_OK;
+      break;
+    }
     if ((spins & 63) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(kWatchMicros)) break;
     __builtin_ia32_pause();
   }
@@ -852,12 +856,9 @@ static int replay_rows(nt_exec* x, int grid, uint64_t paths, uint64_t offset, ui
       if (rc != NT_OK) return rc;
     }
   }
-  const bool watch = grid <= kWatchBlocks;
-  if (watch) std::fill_n(x->h_rows, static_cast<size_t>(grid) * (nch + 2), kUnwritten);
+  std::fill_n(x->h_rows, static_cast<size_t>(grid) * (nch + 2), kUnwritten);
   int rc = ntr::launch_kernel_on(x, x->stream, x->fn, nullptr, d_in, x->d_partials, nch, x->d_scratch, x->d_flags,
-                                 paths, offset, seed,
-                                 reinterpret_cast<double*>(reinterpret_cast<uintptr_t>(x->h_rows) | (watch ? 1 : 0)),
-                                 nullptr, grid);
+                                 paths, offset, seed, reinterpret_cast<double*>(x->h_rows), nullptr, grid);
   if (rc == NT_OK) rc = ntr::await_rows(x, grid);
   if (rc != NT_OK) return rc;
   double replay_ms = 0;

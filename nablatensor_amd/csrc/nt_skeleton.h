@@ -614,22 +614,18 @@ __device__ __forceinline__ void nt_block_store(const double (&acc)[NCH], double*
 // then its NCH sums. The host adds them in nt_finish's order, which saves a
 // small dispatch the second launch, the events around it and its wait for the
 // first (the partials are there too, for when the exception kernel has to
-// run). The lowest bit of `rows` says that the host watches for the words one
-// by one while the kernel ends: each is then a store of its own to system
-// scope. Otherwise the host reads them after the kernel's end, and a wave's
-// plain stores leave as whole lines (391 blocks of 9 words: 97 us per weekday
-// Asian dispatch against 102). The waves' bad lanes meet through `lds`, which
-// holds (NCH + 1) * (blockDim.x / 64) doubles: a __syncthreads_or (256 bytes
-// of LDS and its own reduction) took the fp32 Heston kernel from 80 to 86
+// run). The host watches for the words one by one while the kernel ends, so
+// each is a store of its own to system scope. The waves' bad lanes meet through
+// `lds`, which holds (NCH + 1) * (blockDim.x / 64) doubles: a __syncthreads_or
+// (256 bytes of LDS and its own reduction) took the fp32 Heston kernel from 80 to 86
 // VGPRs, six waves to five.
 #ifndef NT_DUMP_PATHS
 #define NT_ROWS 1
 #endif
 __device__ __forceinline__ nt_u64 nt_clock() { return __builtin_amdgcn_s_memrealtime(); }
 template <typename T>
-__device__ __forceinline__ void nt_to_host(T* at, T v, bool watched) {
-  if (watched) __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  else *at = v;
+__device__ __forceinline__ void nt_to_host(T* at, T v) {
+  __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 template <int NCH>
 __device__ __forceinline__ void nt_block_out(const double (&acc)[NCH], double* __restrict__ partials, double* lds,
@@ -645,21 +641,19 @@ __device__ __forceinline__ void nt_block_out(const double (&acc)[NCH], double* _
   const nt_u64 bad_lanes = __ballot(bad);
   if (lane == 0) lds[NCH * waves + wave] = bad_lanes != 0 ? 1.0 : 0.0;
   __syncthreads();
-  const bool watched = (reinterpret_cast<nt_u64>(rows) & 1) != 0;
-  double* row = reinterpret_cast<double*>(reinterpret_cast<nt_u64>(rows) & ~1ull) +
-                static_cast<nt_u64>(blockIdx.x) * (NCH + 2);
+  double* row = rows + static_cast<nt_u64>(blockIdx.x) * (NCH + 2);
   double* slot = partials + nt_partial_slot(blockIdx.x, gridDim.x);
   for (int c = threadIdx.x; c < NCH; c += blockDim.x) {
     double s = 0.0;
     for (int w = 0; w < waves; ++w) s += lds[c * waves + w];
     slot[c * nt_partial_column(gridDim.x)] = s;
-    if (rows) nt_to_host(row + 2 + c, s, watched);
+    if (rows) nt_to_host(row + 2 + c, s);
   }
   if (rows && threadIdx.x == 0) {
     double any = 0.0;
     for (int w = 0; w < waves; ++w) any += lds[NCH * waves + w];
-    nt_to_host(reinterpret_cast<nt_u64*>(row), started, watched);
-    nt_to_host(reinterpret_cast<nt_u64*>(row) + 1, (nt_clock() << 1) | (any > 0.0 ? 1 : 0), watched);
+    nt_to_host(reinterpret_cast<nt_u64*>(row), started);
+    nt_to_host(reinterpret_cast<nt_u64*>(row) + 1, (nt_clock() << 1) | (any > 0.0 ? 1 : 0));
   }
 }
 

@@ -1,10 +1,11 @@
 """Dispatches whose blocks' sums the host adds (at most 512 blocks) against the
 finishing kernel's sums of the same paths, bit for bit: a one-set
 nt_exec_replay_many, which always runs that kernel. Path counts around a
-block, around the 128 blocks whose rows the host watches for and around the
+block, around 128 blocks and around the
 512-block limit; lanes left to the exception kernel; the reverse sweep; two
 outputs; more channels than a wave has lanes; inputs bound before every call,
-once for several, and changed between calls of both kinds."""
+once for several, and changed between calls of both kinds. Around the limit of
+4,608 words of rows too: 384 blocks of a Heston tape's 12, 124 of a basket's 37."""
 from __future__ import annotations
 
 import numpy as np
@@ -12,6 +13,7 @@ import pytest
 
 from test_gpu_parity import MERTON
 from conftest import equity_tape, merton_call_tape, two_output_tape
+from nablatensor_amd import workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -44,6 +46,13 @@ def tape_of(nt, name):
         return two_output_tape(nt).flat()
     if name == "wide":
         return wide_tape(nt)
+    if name == "heston":
+        return nt.record(nt.HestonModel.asian(nt.OptionTypeEnum.CALL, 1.0, 16), nt.HestonMarket.create(
+            spot=100, strike=100, rate=0.03, v0=0.04, kappa=2.0, theta=0.04, xi=0.5, rho=-0.7)).flat()
+    if name == "basket":
+        fx = workloads.worst_of_inputs()
+        return nt.record(nt.WorstOfBasket.call(fx["corr"], 100.0, 1.0, 16),
+                         nt.WorstOfBasket.market([100.0] * 16, fx["sigma"], 0.03)).flat()
     steps = 1 if name == "european" else 16
     return equity_tape(nt, nt.Products.europeanCall() if steps == 1 else nt.Products.asianCall(),
                        nt.EquityMarket.atmOneYear(), steps).flat()
@@ -64,6 +73,19 @@ def test_small_dispatch_sums_equal_the_finishing_kernels(nt, rocm, name, precisi
                 sums, tm = x.replay(paths, 17, 5)
                 assert np.array_equal(sums, many[0]), (paths, again)
                 assert 0.0 < tm["replay_ms"] <= tm["kernel_ms"] <= tm["wall_ms"]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("name,blocks", [("heston", [128, 383, 384, 385]), ("basket", [123, 124, 125])])
+def test_small_dispatches_around_the_limit_in_words(nt, rocm, name, blocks, precision):
+    flat = tape_of(nt, name)
+    x0 = np.array(flat["recorded_inputs"])
+    with rocm.Executable(flat, rocm.options(precision)) as x:
+        x.set_inputs(x0)
+        for b in blocks:
+            print(f"case {name} {precision} blocks={b}", flush=True)
+            many, _ = x.replay_many(x0[None, :], b * 256 - 3, 17, 5)
+            assert np.array_equal(x.replay(b * 256 - 3, 17, 5)[0], many[0]), b
 
 
 def test_small_dispatch_with_exception_lanes(nt, rocm):
@@ -93,22 +115,19 @@ def test_inputs_changed_between_small_and_large_dispatches(nt, rocm):
             assert np.array_equal(x.replay(1_000, 0, 9)[0], want[1_000][m]), (m, n)
 
 
-def test_watched_dispatches_are_drained(nt, rocm):
-    """A dispatch whose rows the host watches for returns without waiting for the
-    stream, at most 255 times running; any other dispatch waits for it."""
+def test_small_dispatches_are_drained(nt, rocm):
+    """A small dispatch returns without waiting for the stream, at most 255 times
+    running; any other dispatch waits for it."""
     import ctypes as C
     undrained = rocm.lib().nt_testing_undrained
     undrained.argtypes, undrained.restype = [C.c_void_p], C.c_int32
     with rocm.Executable(tape_of(nt, "european"), rocm.options("fp64")) as x:
         seen = []
-        print("case 600 watched dispatches", flush=True)
+        print("case 600 small dispatches", flush=True)
         for k in range(600):
             x.replay(1_000, k * 1_000, 5)
             seen.append(undrained(x._h))
         # one more each time, zero after 255 or where the sums took longer than the host watches
         assert all(b == (a + 1 if a < 255 else 0) or b == 0 for a, b in zip(seen, seen[1:])) and max(seen) <= 255
-        x.replay(200 * 256, 0, 5)  # too many blocks to watch for
-        assert undrained(x._h) == 0
-        x.replay(1_000, 0, 5)
         x.replay(600 * 256, 0, 5)  # the finishing kernel adds these
         assert undrained(x._h) == 0
