@@ -13,7 +13,7 @@
 #define __global__
 #define __device__
 #define __forceinline__ inline
-#define __launch_bounds__(n)
+#define __launch_bounds__(...)
 #define __shared__ static
 #define __constant__ static
 inline void __syncthreads() {}

@@ -87,6 +87,25 @@ def test_draw_sums_match_the_oracle(nt, assets, draws, steps, form, precision):
         assert rel_err(v, ov) < 2e-4 and rel_err(g, og) < 2e-3
 
 
+@pytest.mark.parametrize("basis", [1, 2])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("assets,draws,steps,form", CASES[1::2])
+def test_values_after_the_loop_emitted_on_first_use(nt, assets, draws, steps, form, precision, basis):
+    """Kernels asked for two waves compute each set-up and final value after the
+    loop where it is first read (over inputs and over parameters): the values
+    of the kernels that compute them all at once, bit for bit."""
+    from nablatensor_amd import rocm
+    flat = basket(nt, assets, draws, steps, form)
+    n = len(flat["input_node"])
+    rows = []
+    for waves in (0, 2):
+        src = rocm.lower(flat, rocm.options(precision, mode=2, basis=basis, waves=waves))
+        _, v, g = emu.EmulatedKernel(src, n, tape_slots(src)).run(flat["recorded_inputs"], 150, OFFSET, 42, grid=2, block=64)
+        rows.append((src, v, g))
+    assert rows[0][0] != rows[1][0]
+    assert np.array_equal(rows[0][1], rows[1][1]) and np.array_equal(rows[0][2], rows[1][2])
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_only_the_forms_are_evaluated_on_the_sums(nt, precision):
     """After the loop the step's form is taken on the draws' sums; the exponent and
