@@ -936,8 +936,12 @@ void choose_mode(const TapeIR& t, const nt_options& o, Plan& p) {
   // tangent kernel's time on MI355X: it holds a segment's values, its
   // adjoints and the accumulators at once (more VGPRs, fewer resident waves)
   // and stores and reloads checkpoints. Measured time over (forward +
-  // estimate), reverse against tangent: 1.9-2.2 near the modes' crossover on
-  // the local-volatility Asian (8 to 16 coefficients), 1.3-1.7 on C2-C4.
+  // estimate), reverse against tangent, on the local-volatility Asian: 1.5 to 1.8
+  // at 2 to 16 coefficients and 2.0 at 20 and 24 in fp64, where the modes cross
+  // between 10 (reverse 4.82 ms, tangent 4.76) and 11 (4.95 and 5.24) and this
+  // line lies between 11 and 12; 1.3 to 1.4 at 8 to 12 in fp32, where the
+  // reverse sweep is the faster one already at 8 (1.48 and 1.79 ms) and the line
+  // lies between 10 and 11. On C2-C4 1.3-1.7, far from the line.
   constexpr double kReverseTime = 2.0;
   const bool tangent = o.mode == NT_MODE_TANGENT || p.markets > 1 || multi || price_only ||
                        (p.adjoints && o.mode == NT_MODE_AUTO && fwd + tan < kReverseTime * (fwd + rev));
@@ -1340,16 +1344,21 @@ class Emitter {
   // step's normals): the form of the draws' sums is the sum of the forms, so
   // the loop adds up the draws alone, without the nodes that only feed such
   // exponents (hoist_), and the forms are evaluated once, after the loop, on
-  // those sums (hoisted_step). For a worst-of basket of 16 assets that takes the 136 fma
-  // of the step's 16 x 16 triangular map out of the loop: 2.55 -> 1.89 ms
-  // (fp32) and 6.63 -> 5.02 ms (fp64) per 10^6 paths of 252 steps. Taken when
+  // those sums (hoisted_step). For a worst-of basket of 16 assets that takes the
+  // 136 fma of the step's 16 x 16 triangular map out of the loop: 2.55 -> 1.89 ms
+  // (fp32) and 6.63 -> 4.84 ms (fp64) per 10^6 paths of 252 steps. Taken when
   // it saves at least kSumSaves instructions per step (the carries' sums and
-  // the map's sums against the draws to add); below that, a basket of two, the
-  // draws themselves are nearly all of the step. fp32 sums run over kSumSteps
-  // steps at a time and go to fp64 sums between (a conversion and an add per
-  // draw every kSumSteps steps, under 1 % of them): two assets' paths that end
-  // close to each other keep their order, which decides the asset a worst-of
-  // credits its derivatives to.
+  // the map's sums against the draws to add): three assets are the smallest
+  // basket that does; for two, the draws are nearly all of the step. The running
+  // sums hold registers, a wave or two fewer for most baskets below 16, and
+  // the loop is still faster at each size (us per 3x10^5 paths, before -> with):
+  // 3 assets 143 -> 134 (fp32) and 325 -> 279 (fp64), 4: 186 -> 170 and 429 ->
+  // 363, 6: 267 -> 242 and 641 -> 532, 8: 371 -> 316 and 847 -> 658, 12: 549 ->
+  // 471 and 1,336 -> 965, 15: 775 -> 578 and 2,002 -> 1,506. fp32 sums run over
+  // kSumSteps steps at a time and go to fp64 sums between (a conversion and an
+  // add per draw every kSumSteps steps, under 1 % of them): two assets' paths
+  // that end close to each other keep their order, which decides the asset a
+  // worst-of credits its derivatives to.
   static constexpr int kSumSaves = 4;
   static constexpr int kSumSteps = 16;
   // per loop position: a draw summed over the loop; a node the loop does not

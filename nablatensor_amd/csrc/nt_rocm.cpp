@@ -451,8 +451,8 @@ namespace ntr {
 // in device memory sizes that tape per lane of the largest grid, so it gets
 // the larger grid only while the tape stays within kTapeBudget, and only with
 // two or more waves per SIMD resident: at one wave per SIMD its tape traffic,
-// not the tail, sets the time (local-volatility tape, 388 VGPRs: 8.89 ms
-// resident, 9.33 ms on 8 resident grids).
+// not the tail, sets the time (local-volatility tape, 336 VGPRs: 7.25 ms
+// resident, 7.92 ms on 2, 4 and 8 resident grids).
 // Whole blocks per CU matter as much as the count: a grid of q CUs' worth
 // plus r blocks leaves r CUs one block longer than the rest. Measured on one
 // MI355X (bench.py --max-blocks, two runs per grid, kernel HIP-event means),

@@ -237,9 +237,11 @@ __device__ __forceinline__ double nt_exp(double x) {
 #ifdef NT_TURN_DRAWS
 // The routines of tapes whose step takes the square root of an active value (a
 // variance): near its floor such a value multiplies the last bit of a draw by
-// 1 / (2 sqrt v), and one path of 10^7 can move a derivative's sum by 3e-11 of
-// itself. These tapes keep the rounding of their draws and roots, from the
-// routines below; every other tape takes the shorter ones after them.
+// 1 / (2 sqrt v), and with the shorter routines one path of 10^7 moved a
+// derivative's sum by 3e-11 of itself from the result with these (which of the
+// two lies nearer the exact sum was not measured). These tapes keep the rounding
+// of their draws and roots, from the routines below; every other tape takes the
+// shorter ones after them.
 
 // -2 ln(u) for a positive normal u, by Tang's method with F = x rounded to 8
 // fractional bits of its binade and r = (x - F) / F, x - F exact.
