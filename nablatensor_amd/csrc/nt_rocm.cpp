@@ -354,8 +354,7 @@ int decline_spill(const nt_exec_info& info, const nt_options* opt) {
 // steps: 273 and 276 VGPRs, one wave, 1.24 and 2.25 ms; 158 and 195 VGPRs, 1.05
 // and 1.50 ms). An explicit nt_options.waves is left as asked.
 constexpr int kSecondWaveReverse = 16, kSecondWaveTangent = 32;
-int compile_replay(const nt_tape* tape, const nt_options* options, Lowered& low, std::vector<char>& code,
-                   nt_exec_info& info) {
+int compile_replay(const nt_options* options, Lowered& low, std::vector<char>& code, nt_exec_info& info) {
   double secs = 0;
   int rc = compile_hiprtc(low.source, false, code, secs);
   if (rc != NT_OK) return rc;
@@ -365,22 +364,23 @@ int compile_replay(const nt_tape* tape, const nt_options* options, Lowered& low,
   const bool asked = options && options->waves > 0;
   const int over = low.plan.mode == NT_MODE_TANGENT ? kSecondWaveTangent : kSecondWaveReverse;
   if (asked || info.vgprs <= 256 || info.vgprs > 256 + over) return NT_OK;
-  nt_options o = options ? *options : nt_options{};
-  o.waves = 2;
-  Lowered low2;
+  // The plan does not depend on the waves asked for (60 of the 66 ms that the
+  // 16-asset worst-of takes to lower), so only the source is emitted again.
+  ntl::Plan plan2 = low.plan;
+  plan2.waves = 2;
+  std::string source2 = ntl::emit_source(low.ir, plan2);
   std::vector<char> code2;
   double secs2 = 0;
-  if (lower(tape, &o, low2) != NT_OK || compile_hiprtc(low2.source, false, code2, secs2) != NT_OK) {
+  if (compile_hiprtc(source2, false, code2, secs2) != NT_OK) {
     (void)fail(NT_OK, std::string());  // the first compile stands; drop the retry's message
     return NT_OK;
   }
-  nt_exec_info info2{};
-  fill_static_info(low2, info2);
-  kernel_resources(code2, "nt_replay", info2);
   info.compile_seconds += secs2;
+  nt_exec_info info2 = info;
+  kernel_resources(code2, "nt_replay", info2);
   if (info2.scratch_bytes != 0 || info2.vgprs < 0 || info2.vgprs > 256) return NT_OK;
-  info2.compile_seconds = info.compile_seconds;
-  low = std::move(low2);
+  low.plan = std::move(plan2);
+  low.source = std::move(source2);
   code = std::move(code2);
   info = info2;
   return NT_OK;
@@ -683,7 +683,7 @@ int nt_compile_check(const nt_tape* tape, const nt_options* options, nt_exec_inf
   if (rc != NT_OK) return rc;
   std::vector<char> code;
   nt_exec_info res{};
-  rc = compile_replay(tape, options, l, code, res);
+  rc = compile_replay(options, l, code, res);
   if (rc != NT_OK) return rc;
   if (info) *info = res;
   return decline_spill(res, options);
@@ -701,7 +701,7 @@ int nt_exec_create(const nt_tape* tape, const nt_options* options, nt_exec** out
   if (rc != NT_OK) return rc;
   rc = device_index(x->dev);
   if (rc != NT_OK) return rc;
-  rc = compile_replay(tape, options, x->low, x->code, x->info);
+  rc = compile_replay(options, x->low, x->code, x->info);
   if (rc != NT_OK) return rc;
   rc = decline_spill(x->info, options);
   if (rc != NT_OK) return rc;
