@@ -1,11 +1,11 @@
 """Dispatches whose blocks' sums the host adds (at most 512 blocks) against the
 finishing kernel's sums of the same paths, bit for bit: a one-set
 nt_exec_replay_many, which always runs that kernel. Path counts around a
-block, around 128 blocks and around the
-512-block limit; lanes left to the exception kernel; the reverse sweep; two
-outputs; more channels than a wave has lanes; inputs bound before every call,
-once for several, and changed between calls of both kinds. Around the limit of
-4,608 words of rows too: 384 blocks of a Heston tape's 12, 124 of a basket's 37."""
+block, around 128 blocks and around the 512-block limit, and around the limit
+of 4,608 words of rows (384 blocks of a Heston tape's 12, 124 of a basket's
+37); lanes left to the exception kernel; the reverse sweep; two outputs; more
+channels than a wave has lanes; inputs bound before every call, once for
+several, and changed between calls of both kinds."""
 from __future__ import annotations
 
 import numpy as np
